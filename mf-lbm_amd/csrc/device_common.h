@@ -56,45 +56,30 @@ __device__ __forceinline__ int link_slot(int nc, const int* wbase, const unsigne
 // The odd step's neighbour slots of fluid node m (compact index; m & 63 its lane, every lane of the wave in one link
 // mask word) at dense offset n: per direction r, the index of the slot (x + e_r, opp(r)) in slice opp(r), which is
 // the link slot of (m, r) where the wave's link mask has m's bit, else the compact index of the fluid node x + e_r.
-// The wave-uniform masks and bases are scalar loads issued together; x + e_r lies inside the padded grid, so the
-// 18 dense map entries are loaded unconditionally, all in flight at once, and selected afterwards (a conditional
-// load per direction compiles to a branch that waits for every earlier load).  ROWS: the entries of a row of three
-// directions (ex = -1, 0, +1 at one (ey, ez)) are adjacent and taken by one 12-byte load (10 load instructions
-// instead of 18): 1.6-2.1 % faster single-phase steps at 256^3, 0.4 % slower for the two-phase update, whose
-// curvature stencil keeps more loads in flight.
-template <bool ROWS>
-__device__ __forceinline__ void odd_neighbour_slots(const int* __restrict__ map, const Layout& L, int nc,
+// The wave-uniform masks and bases are scalar loads issued together; the eight row records around the node's own row
+// (layout.h) are loaded unconditionally, all in flight at once (a conditional load per direction compiles to a branch
+// that waits for every earlier load), and every fluid neighbour's index is its row's rank or one next to it.
+__device__ __forceinline__ void odd_neighbour_slots(const RowRec* __restrict__ rows, const Layout& L, int nc,
                                                     const int* __restrict__ wbase,
                                                     const unsigned long long* __restrict__ wmask, int m, int n,
                                                     unsigned nb[19]) {
     const int e0 = 18 * __builtin_amdgcn_readfirstlane(m >> 6) - 1;
     const unsigned lane = (unsigned)m & 63u;
     const unsigned long long below = (1ull << lane) - 1ull;
-    unsigned mv[19];
-    if constexpr (ROWS) {   // rows (ey, ez) = (0, 0), (1, 0), (-1, 0), (0, 1), (0, -1); the four directions with ey
-                            // and ez both nonzero one by one (4-byte aligned 12-byte loads)
-        struct __attribute__((aligned(4))) Row {
-            int v[3];
-        };
-        Row row[5];
-        const int rb[5] = {n - 1, n + L.px - 1, n - L.px - 1, n + L.pxy - 1, n - L.pxy - 1};
+    const int g = n >> 4, sx = L.px >> 4, sxy = L.pxy >> 4;
+    RowRec row[9];   // entry 3 (ez + 1) + ey + 1
 #pragma unroll
-        for (int k = 0; k < 5; ++k) row[k] = *(const Row*)(map + rb[k]);
-#pragma unroll
-        for (int r = 1; r < 19; ++r) {
-            const int ey = lat::EY[r], ez = lat::EZ[r];
-            const int k = ey == 1 ? 1 : ey == -1 ? 2 : ez == 1 ? 3 : ez == -1 ? 4 : 0;
-            mv[r] = (unsigned)((ey != 0 && ez != 0) ? map[n + L.off(r)] : row[k].v[lat::EX[r] + 1]);
-        }
-    } else {
-#pragma unroll
-        for (int r = 1; r < 19; ++r) mv[r] = (unsigned)map[n + L.off(r)];
-    }
+    for (int k = 0; k < 9; ++k)
+        if (k != 4) row[k] = rows[g + (k % 3 - 1) * sx + (k / 3 - 1) * sxy];
 #pragma unroll
     for (int r = 1; r < 19; ++r) {
+        const int ex = lat::EX[r], k = 3 * (lat::EZ[r] + 1) + lat::EY[r] + 1;
+        unsigned mv;
+        if (k == 4) mv = (unsigned)(m + ex);
+        else mv = row_rank(row[k], n) + (ex < 0 ? ~0u : ex > 0 ? row_fluid(row[k], n, 0) : 0u);
         const unsigned long long wm = wmask[e0 + r];
         const unsigned li = (unsigned)(nc + wbase[e0 + r]) + (unsigned)__popcll(wm & below);
-        nb[r] = ((wm >> lane) & 1ull) ? li : mv[r];
+        nb[r] = ((wm >> lane) & 1ull) ? li : mv;
     }
 }
 

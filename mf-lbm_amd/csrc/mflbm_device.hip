@@ -48,6 +48,7 @@ struct Dev {
     const int* map;   // padded offset -> compact index, -1 where nothing is stored
     const int* pmap;  // padded offset -> compact index of an interior fluid node, -1 elsewhere (a folded halo node
                       // maps to its image in map but not here: its phi is the dense one the periodic copy writes)
+    const RowRec* rows;   // row records (layout.h)
     const int* cpos;  // compact index -> padded offset
     int nf;           // interior fluid nodes
     int nc;           // all compact nodes
@@ -335,7 +336,7 @@ k_collide(Dev d, CollideParams P, int per) {
         b[0] = v.y;
     }
     if (ODD) {
-        odd_neighbour_slots<false>(d.map, d.L, d.nc, d.wbase, d.wmask, m, nn, nb);
+        odd_neighbour_slots(d.rows, d.L, d.nc, d.wbase, d.wmask, m, nn, nb);
 #pragma unroll
         for (int q = 1; q < 19; ++q) {   // slot q of the upwind node x - e_q = x + e_opp(q)
             const double2 v = ld_pair(S.p[q], nb[lat::OPP[q]]);
@@ -400,7 +401,7 @@ __global__ void __launch_bounds__(BLOCK) k_collide32(Dev d, CollideParamsDev<C> 
         a[0] = v.y;
     }
     if (ODD) {
-        odd_neighbour_slots<false>(d.map, d.L, d.nc, d.wbase, d.wmask, m, nn, nb);
+        odd_neighbour_slots(d.rows, d.L, d.nc, d.wbase, d.wmask, m, nn, nb);
 #pragma unroll
         for (int q = 1; q < 19; ++q) {
             const float2 v = ld_pair32(S.p[q], nb[lat::OPP[q]]);
@@ -2017,6 +2018,7 @@ struct mflbm_ctx {
     bool fp32 = false;          // precision 1 or 2: FP32 storage (s, a) of collide.h
     double* force = nullptr;    // 4 compact force arrays
     int* map = nullptr;         // Dev::map, then Dev::pmap (2 x L.total)
+    RowRec* rows = nullptr;     // Dev::rows
     int* ibuf = nullptr;        // cpos, normal list, solid lists, fluid list positions
     int* wbuf = nullptr;        // per normal-list node: index into the fluid boundary list or -1
     unsigned* mbuf = nullptr;   // solid list masks
@@ -2320,12 +2322,13 @@ int scatter_state(mflbm_ctx* c) {
 }
 
 void free_geometry(mflbm_ctx* c) {
-    void* bufs[] = {c->compact, c->force, c->map, c->ibuf, c->wbuf, c->mbuf, c->dbuf, c->wmask, c->wbase, c->role, c->qbuf, c->cbuf, c->phic};
+    void* bufs[] = {c->compact, c->force, c->map, c->rows, c->ibuf, c->wbuf, c->mbuf, c->dbuf, c->wmask, c->wbase, c->role, c->qbuf, c->cbuf, c->phic};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     c->compact = nullptr;
     c->force = nullptr;
     c->map = nullptr;
+    c->rows = nullptr;
     c->ibuf = nullptr;
     c->wbuf = nullptr;
     c->mbuf = nullptr;
@@ -2615,6 +2618,12 @@ extern "C" int mflbm_upload_geometry(mflbm_ctx* c, const int8_t* walls_h2, int32
         for (int m = 0; m < nfl; ++m) pm[cpos[m]] = m;
         HIPCHK(c, hipMemcpy(c->map + L.total, pm.data(), sizeof(int) * L.total, hipMemcpyHostToDevice));
     }
+    {
+        std::vector<RowRec> rows;
+        build_rows(L, cset, rows);
+        HIPCHK(c, hipMalloc(&c->rows, sizeof(RowRec) * rows.size()));
+        HIPCHK(c, hipMemcpy(c->rows, rows.data(), sizeof(RowRec) * rows.size(), hipMemcpyHostToDevice));
+    }
     HIPCHK(c, hipMalloc(&c->role, sizeof(int) * L.total));
     HIPCHK(c, hipMemcpy(c->role, role.data(), sizeof(int) * L.total, hipMemcpyHostToDevice));
     // brick flags (Dev): notm and notp (two buffers each), bstatic, nzb, nzd.  The band flags, nzb and nzd start
@@ -2683,6 +2692,7 @@ extern "C" int mflbm_upload_geometry(mflbm_ctx* c, const int8_t* walls_h2, int32
     }
     d.map = c->map;
     d.pmap = c->map + L.total;
+    d.rows = c->rows;
     d.phic = c->phic;
     d.cpos = c->ibuf;
     d.nf = nfl;

@@ -460,6 +460,12 @@ extern "C" int mflbm_spb_commit(mflbm_spb_ctx* c) {
         c->bufs.push_back(wmask);
         HIPCHK(c, hipMalloc(&wbase, sizeof(int) * ls[s].wbase.size()));
         c->bufs.push_back(wbase);
+        std::vector<RowRec> hrows;
+        build_rows(L, cs[s], hrows);
+        RowRec* rows = nullptr;
+        HIPCHK(c, hipMalloc(&rows, sizeof(RowRec) * hrows.size()));
+        c->bufs.push_back(rows);
+        HIPCHK(c, hipMemcpy(rows, hrows.data(), sizeof(RowRec) * hrows.size(), hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(map, cs[s].cidx.data(), sizeof(int) * L.total, hipMemcpyHostToDevice));
         if (c->nc[s] > 0) HIPCHK(c, hipMemcpy(cpos, cs[s].cpos.data(), sizeof(int) * c->nc[s], hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(wmask, ls[s].wmask.data(), sizeof(unsigned long long) * ls[s].wmask.size(), hipMemcpyHostToDevice));
@@ -467,6 +473,7 @@ extern "C" int mflbm_spb_commit(mflbm_spb_ctx* c) {
         const long* so = &c->soff[20L * s];
         d64[s].L = L;
         d64[s].map = map;
+        d64[s].rows = rows;
         d64[s].cpos = cpos;
         d64[s].nf = c->nf[s];
         d64[s].nc = c->nc[s];
@@ -477,6 +484,7 @@ extern "C" int mflbm_spb_commit(mflbm_spb_ctx* c) {
         d64[s].cf = nullptr;
         d32[s].L = L;
         d32[s].map = map;
+        d32[s].rows = rows;
         d32[s].cpos = cpos;
         d32[s].nf = c->nf[s];
         d32[s].nc = c->nc[s];

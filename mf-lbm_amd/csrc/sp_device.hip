@@ -277,6 +277,7 @@ struct mflbm_sp_ctx {
     double* red = nullptr;       // monitor layer results (3*nz)
     void* compact = nullptr;     // 19 population slices (compact slots + link slots), double or float
     int* map = nullptr;
+    RowRec* rows = nullptr;
     int* cpos = nullptr;
     unsigned long long* wmask = nullptr;
     int* wbase = nullptr;
@@ -403,11 +404,12 @@ int sp_macro_t(mflbm_sp_ctx* c) {
 }
 
 void sp_free_geometry(mflbm_sp_ctx* c) {
-    void* bufs[] = {c->compact, c->map, c->cpos, c->wmask, c->wbase};
+    void* bufs[] = {c->compact, c->map, c->rows, c->cpos, c->wmask, c->wbase};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     c->compact = nullptr;
     c->map = nullptr;
+    c->rows = nullptr;
     c->cpos = nullptr;
     c->wmask = nullptr;
     c->wbase = nullptr;
@@ -550,6 +552,12 @@ extern "C" int mflbm_sp_upload_geometry(mflbm_sp_ctx* c, const int8_t* walls_h2,
     HIPCHK(c, hipMemset(c->compact, 0, esz * soff[19]));
     HIPCHK(c, hipMemset(c->fields, 0, sizeof(double) * c->ps * 4));
     HIPCHK(c, hipMemcpy(c->map, cset.cidx.data(), sizeof(int) * L.total, hipMemcpyHostToDevice));
+    {
+        std::vector<RowRec> rows;
+        build_rows(L, cset, rows);
+        HIPCHK(c, hipMalloc(&c->rows, sizeof(RowRec) * rows.size()));
+        HIPCHK(c, hipMemcpy(c->rows, rows.data(), sizeof(RowRec) * rows.size(), hipMemcpyHostToDevice));
+    }
     if (nc > 0) HIPCHK(c, hipMemcpy(c->cpos, cset.cpos.data(), sizeof(int) * nc, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->wmask, links.wmask.data(), sizeof(unsigned long long) * links.wmask.size(), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->wbase, links.wbase.data(), sizeof(int) * links.wbase.size(), hipMemcpyHostToDevice));
@@ -562,6 +570,7 @@ extern "C" int mflbm_sp_upload_geometry(mflbm_sp_ctx* c, const int8_t* walls_h2,
         d32.S[q] = c->fp32 ? (float*)c->compact + soff[q] : nullptr;
     }
     d.map = d32.map = c->map;
+    d.rows = d32.rows = c->rows;
     d.cpos = d32.cpos = c->cpos;
     d.nf = d32.nf = cset.nfl;
     d.nc = d32.nc = nc;
