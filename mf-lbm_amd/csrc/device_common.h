@@ -53,16 +53,21 @@ __device__ __forceinline__ int link_slot(int nc, const int* wbase, const unsigne
     return nc + wbase[e] + __popcll(wm & ((1ull << l) - 1ull));
 }
 
+// A pointer that a kernel read from memory is generic to the compiler: accesses through it are flat instructions with a
+// 64-bit vector address each.  Named as global it takes the scalar-base form that a kernel argument gets by itself.
+#define MFLBM_GLOBAL __attribute__((address_space(1)))
+
 // The odd step's neighbour slots of fluid node m (compact index; m & 63 its lane, every lane of the wave in one link
 // mask word) at dense offset n: per direction r, the index of the slot (x + e_r, opp(r)) in slice opp(r), which is
 // the link slot of (m, r) where the wave's link mask has m's bit, else the compact index of the fluid node x + e_r.
 // The wave-uniform masks and bases are scalar loads issued together; the eight row records around the node's own row
 // (layout.h) are loaded unconditionally, all in flight at once (a conditional load per direction compiles to a branch
 // that waits for every earlier load), and every fluid neighbour's index is its row's rank or one next to it.
-__device__ __forceinline__ void odd_neighbour_slots(const RowRec* __restrict__ rows, const Layout& L, int nc,
-                                                    const int* __restrict__ wbase,
-                                                    const unsigned long long* __restrict__ wmask, int m, int n,
-                                                    unsigned nb[19]) {
+__device__ __forceinline__ void odd_neighbour_slots(const RowRec* rows_, const Layout& L, int nc, const int* wbase_,
+                                                    const unsigned long long* wmask_, int m, int n, unsigned nb[19]) {
+    const MFLBM_GLOBAL long* const rows = (const MFLBM_GLOBAL long*)rows_;
+    const MFLBM_GLOBAL int* const wbase = (const MFLBM_GLOBAL int*)wbase_;
+    const MFLBM_GLOBAL unsigned long long* const wmask = (const MFLBM_GLOBAL unsigned long long*)wmask_;
     const int e0 = 18 * __builtin_amdgcn_readfirstlane(m >> 6) - 1;
     const unsigned lane = (unsigned)m & 63u;
     const unsigned long long below = (1ull << lane) - 1ull;
@@ -70,7 +75,7 @@ __device__ __forceinline__ void odd_neighbour_slots(const RowRec* __restrict__ r
     RowRec row[9];   // entry 3 (ez + 1) + ey + 1
 #pragma unroll
     for (int k = 0; k < 9; ++k)
-        if (k != 4) row[k] = rows[g + (k % 3 - 1) * sx + (k / 3 - 1) * sxy];
+        if (k != 4) row[k] = __builtin_bit_cast(RowRec, rows[g + (k % 3 - 1) * sx + (k / 3 - 1) * sxy]);
 #pragma unroll
     for (int r = 1; r < 19; ++r) {
         const int ex = lat::EX[r], k = 3 * (lat::EZ[r] + 1) + lat::EY[r] + 1;
@@ -87,11 +92,11 @@ __device__ __forceinline__ void odd_neighbour_slots(const RowRec* __restrict__ r
 // base instead of a 64-bit vector address per slot); slices are kept below 2^32 bytes.
 template <class T>
 __device__ __forceinline__ T slot_ld(const T* slice, unsigned i) {
-    return *(const T*)((const char*)slice + i * (unsigned)sizeof(T));
+    return *(const MFLBM_GLOBAL T*)((const MFLBM_GLOBAL char*)slice + i * (unsigned)sizeof(T));
 }
 template <class T>
 __device__ __forceinline__ void slot_st(T* slice, unsigned i, T v) {
-    *(T*)((char*)slice + i * (unsigned)sizeof(T)) = v;
+    *(MFLBM_GLOBAL T*)((MFLBM_GLOBAL char*)slice + i * (unsigned)sizeof(T)) = v;
 }
 
 // Exchanged halo slots of a folded domain (layout.h, Fold): the halo slot (q, h) of a direction q that points

@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(NT) k_spb_collide(const SDev<T>* __restrict__ 
     if (w >= nwaves) return;
     const int s = __builtin_amdgcn_readfirstlane(wave_sample[w]);
     if (!active[s]) return;
-    const SDev<T>& d = devs[s];
+    const SDev<T> d = devs[s];   // a copy: the slice bases stay scalar across the stores
     const int m = (w - wave_first[s]) * WAVE + (int)(threadIdx.x % WAVE);
     if (m >= d.nf) return;
     sp_update_node<ODD, T, C>(d, P, m);
