@@ -33,7 +33,7 @@ inline Layout make_layout(int nx, int ny, int nz) {
     return L;
 }
 
-// copy between the reference's halo-h layout (host) and the padded device layout (one array)
+// copy from the reference's halo-h layout (host) into the padded device layout (one array)
 template <typename T>
 void pack_host(const Layout& L, int h, const T* src, T* dst_padded) {
     const int sx = L.nx + 2 * h, sy = L.ny + 2 * h;
@@ -41,15 +41,6 @@ void pack_host(const Layout& L, int h, const T* src, T* dst_padded) {
         for (int j = 1 - h; j <= L.ny + h; ++j) {
             const T* s = src + (long)(j + h - 1) * sx + (long)(k + h - 1) * sx * sy;
             std::memcpy(dst_padded + L.at(1 - h, j, k), s, sizeof(T) * sx);
-        }
-}
-template <typename T>
-void unpack_host(const Layout& L, int h, const T* src_padded, T* dst) {
-    const int sx = L.nx + 2 * h, sy = L.ny + 2 * h;
-    for (int k = 1 - h; k <= L.nz + h; ++k)
-        for (int j = 1 - h; j <= L.ny + h; ++j) {
-            T* d = dst + (long)(j + h - 1) * sx + (long)(k + h - 1) * sx * sy;
-            std::memcpy(d, src_padded + L.at(1 - h, j, k), sizeof(T) * sx);
         }
 }
 

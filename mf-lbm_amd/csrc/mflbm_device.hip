@@ -21,6 +21,7 @@
 
 #include "collide.h"
 #include "device_common.h"
+#include "download.h"
 #include "lattice.h"
 #include "mflbm.h"
 
@@ -1832,7 +1833,7 @@ __global__ void k_zero_solid_phi(Dev d) {
 }
 // one block per z layer: the seven layer sums of Monitor.F90:62-84 and per-layer partials of the global
 // scalars, reduced in a fixed tree (deterministic run to run)
-constexpr int NPART = 12;
+constexpr int NPART = 12, NPART_MORE = 4;
 __global__ void __launch_bounds__(BLOCK) k_monitor_layers(Dev d, const double* u, const double* v, const double* w,
                                                            const double* rho, const double* phi_old, double* layers,
                                                            double* part) {
@@ -1865,19 +1866,25 @@ __global__ void __launch_bounds__(BLOCK) k_monitor_layers(Dev d, const double* u
             dphi = fmax(dphi, fabs(ph - phi_old[n]) * om);
         }
     }
-    // count of fluid-1 nodes (phi > 0.99) for the capillary-pressure monitor
-    double c1 = 0.0;
+    // count of fluid-1 nodes (phi > 0.99) for the capillary-pressure monitor, and of nodes with phi > 0 for the
+    // breakthrough monitor (Monitor.F90:472-507; read at layer nz - 1)
+    double c1 = 0.0, c0 = 0.0;
     for (int r = threadIdx.x; r < nxy; r += BLOCK) {
         const int n = L.at(r % L.nx + 1, r / L.nx + 1, k);
-        if (d.walls[n] == 0 && d.phi[n] > 0.99) c1 += 1.0;
+        if (d.walls[n] == 0) {
+            const double ph = d.phi[n];
+            if (ph > 0.99) c1 += 1.0;
+            if (ph > 0.0) c0 += 1.0;
+        }
     }
     // wavefront reductions (a fixed butterfly over the 64 lanes), then the four waves' results in wave order
-    constexpr int NQ = NPART + 3, NW = BLOCK / 64;
+    constexpr int NQ = NPART + NPART_MORE, NW = BLOCK / 64;
     double q15[NQ];
     for (int m = 0; m < NPART; ++m) q15[m] = s[m];
     q15[NPART] = umax;
     q15[NPART + 1] = dphi;
     q15[NPART + 2] = c1;
+    q15[NPART + 3] = c0;
 #pragma unroll
     for (int m = 0; m < NQ; ++m)
 #pragma unroll
@@ -1899,7 +1906,7 @@ __global__ void __launch_bounds__(BLOCK) k_monitor_layers(Dev d, const double* u
         }
     if (threadIdx.x == 0) {
         for (int m = 0; m < 7; ++m) layers[m * L.nz + (k - 1)] = out[m];
-        for (int m = 7; m < NPART + 3; ++m) part[(m - 7) * L.nz + (k - 1)] = out[m];
+        for (int m = 7; m < NQ; ++m) part[(m - 7) * L.nz + (k - 1)] = out[m];
     }
 }
 // Initial state of a new run at rest, on the device (initialization_new_multi / _pdf, Init_multiphase.F90:
@@ -2013,6 +2020,7 @@ struct mflbm_ctx {
     double* rho = nullptr;
     double* phi_old = nullptr;
     double* red = nullptr;      // monitor layer sums and partials
+    Downloader dl;              // pinned ring of the downloads
     // geometry-dependent device buffers
     void* compact = nullptr;    // 38 population slices (compact slots + link slots), FP64 or FP32
     bool fp32 = false;          // precision 1 or 2: FP32 storage (s, a) of collide.h
@@ -2435,6 +2443,7 @@ extern "C" void mflbm_destroy(mflbm_ctx* c) {
     for (auto e : c->ev)
         if (e) (void)hipEventDestroy(e);
     free_geometry(c);
+    c->dl.free();
     void* bufs[] = {c->dense_pdf, c->fields, c->fields32, c->walls, c->planes, c->red};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
@@ -2812,18 +2821,13 @@ extern "C" int mflbm_download_state(mflbm_ctx* c, double* const* f, double* cons
         const int rr = refresh_solid_phi(c);
         if (rr) return rr;
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    std::vector<double> buf(L.total);
+    std::vector<DownloadItem> items;
     for (int q = 0; q < 38; ++q) {
         double* dst = q < 19 ? (f ? f[q] : nullptr) : (g ? g[q - 19] : nullptr);
-        if (!dst) continue;
-        HIPCHK(c, hipMemcpy(buf.data(), c->dense_pdf + q * c->ps, sizeof(double) * L.total, hipMemcpyDeviceToHost));
-        unpack_host(L, 1, buf.data(), dst);
+        if (dst) items.push_back(DownloadItem{c->dense_pdf + q * c->ps, 0, 1, 1, dst});
     }
-    if (phi) {
-        HIPCHK(c, hipMemcpy(buf.data(), c->d.phi, sizeof(double) * L.total, hipMemcpyDeviceToHost));
-        unpack_host(L, 4, buf.data(), phi);
-    }
+    if (phi) items.push_back(DownloadItem{c->d.phi, 0, 1, 4, phi});
+    HIPCHK(c, c->dl.run(L, c->stream, items));
     const size_t plane = (size_t)(L.nx + 2) * (L.ny + 2);
     if (f_convec) HIPCHK(c, hipMemcpy(f_convec, c->d.cf, sizeof(double) * plane * 19, hipMemcpyDeviceToHost));
     if (g_convec) HIPCHK(c, hipMemcpy(g_convec, c->d.cg, sizeof(double) * plane * 19, hipMemcpyDeviceToHost));
@@ -2883,7 +2887,7 @@ extern "C" int mflbm_monitor(mflbm_ctx* c, double* layers, mflbm_monitor_sums* s
     double* part = c->red + 7 * (size_t)L.nz;
     LAUNCH(c, k_monitor_layers, (unsigned)L.nz, c->d, c->u, c->v, c->w, c->rho, c->phi_old,
            lay, part);
-    std::vector<double> h((size_t)L.nz * (7 + NPART + 3 - 7));
+    std::vector<double> h((size_t)L.nz * (NPART + NPART_MORE));
     HIPCHK(c, hipMemcpyAsync(h.data(), c->red, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (layers) std::memcpy(layers, h.data(), sizeof(double) * 7 * L.nz);
@@ -2904,17 +2908,7 @@ extern "C" int mflbm_monitor(mflbm_ctx* c, double* layers, mflbm_monitor_sums* s
             s.vol1_full += h[2 * (size_t)L.nz + k];
             s.vol2_full += h[3 * (size_t)L.nz + k];
         }
-        // breakthrough count at z = nz-1 (Monitor.F90:472-507)
-        std::vector<double> phil((size_t)L.nx * L.ny);
-        std::vector<int8_t> wl((size_t)L.nx * L.ny);
-        for (int j = 1; j <= L.ny; ++j) {
-            HIPCHK(c, hipMemcpy(phil.data() + (size_t)(j - 1) * L.nx, c->d.phi + L.at(1, j, L.nz - 1), sizeof(double) * L.nx,
-                                hipMemcpyDeviceToHost));
-            HIPCHK(c, hipMemcpy(wl.data() + (size_t)(j - 1) * L.nx, c->walls + L.at(1, j, L.nz - 1), (size_t)L.nx,
-                                hipMemcpyDeviceToHost));
-        }
-        for (size_t m = 0; m < phil.size(); ++m)
-            if (wl[m] == 0 && phil[m] > 0.0) s.outlet_phase1++;
+        s.outlet_phase1 = (int64_t)row(8)[L.nz - 2];   // breakthrough count at z = nz-1
         *sums = s;
     }
     if (update_phi_old) {
@@ -2930,15 +2924,12 @@ extern "C" int mflbm_download_macro(mflbm_ctx* c, double* u, double* v, double* 
         const int rr = refresh_solid_phi(c);
         if (rr) return rr;
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    std::vector<double> buf(L.total);
     double* src[5] = {c->u, c->v, c->w, c->rho, c->d.phi};
     double* dst[5] = {u, v, w, rho, phi};
-    for (int m = 0; m < 5; ++m) {
-        if (!dst[m]) continue;
-        HIPCHK(c, hipMemcpy(buf.data(), src[m], sizeof(double) * L.total, hipMemcpyDeviceToHost));
-        unpack_host(L, m == 4 ? 4 : 1, buf.data(), dst[m]);
-    }
+    std::vector<DownloadItem> items;
+    for (int m = 0; m < 5; ++m)
+        if (dst[m]) items.push_back(DownloadItem{src[m], 0, 1, m == 4 ? 4 : 1, dst[m]});
+    HIPCHK(c, c->dl.run(L, c->stream, items));
     return MFLBM_OK;
 }
 
@@ -2959,28 +2950,14 @@ extern "C" int mflbm_download_gradient(mflbm_ctx* c, double* cn_x, double* cn_y,
         if (c->fp32) LAUNCH(c, k_curvature_dense<float>, nblocks((long)L.nx * L.ny * L.nz), c->d);
         else LAUNCH(c, k_curvature_dense<double>, nblocks((long)L.nx * L.ny * L.nz), c->d);
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    std::vector<double> buf(L.total);
-    double* dst[5] = {cn_x, cn_y, cn_z, c_norm, curv};
-    if (cn_x || cn_y || cn_z || c_norm) {   // the records, split into the components (FP32 widened)
-        std::vector<double> rec(4 * (size_t)L.total);
-        if (c->fp32) {
-            std::vector<float> rec32(4 * (size_t)L.total);
-            HIPCHK(c, hipMemcpy(rec32.data(), c->d.cn32, sizeof(float) * rec32.size(), hipMemcpyDeviceToHost));
-            for (size_t k = 0; k < rec.size(); ++k) rec[k] = (double)rec32[k];
-        } else {
-            HIPCHK(c, hipMemcpy(rec.data(), c->d.cn, sizeof(double) * rec.size(), hipMemcpyDeviceToHost));
-        }
-        for (int m = 0; m < 4; ++m) {
-            if (!dst[m]) continue;
-            for (long k = 0; k < L.total; ++k) buf[k] = rec[4 * (size_t)k + m];
-            unpack_host(L, 2, buf.data(), dst[m]);
-        }
-    }
-    if (curv) {
-        HIPCHK(c, hipMemcpy(buf.data(), c->d.curv, sizeof(double) * L.total, hipMemcpyDeviceToHost));
-        unpack_host(L, 1, buf.data(), curv);
-    }
+    double* dst[4] = {cn_x, cn_y, cn_z, c_norm};   // the components of the records (FP32 widened)
+    std::vector<DownloadItem> items;
+    for (int m = 0; m < 4; ++m)
+        if (dst[m])
+            items.push_back(c->fp32 ? DownloadItem{(const float*)c->d.cn32 + m, 1, 4, 2, dst[m]}
+                                    : DownloadItem{(const double*)c->d.cn + m, 0, 4, 2, dst[m]});
+    if (curv) items.push_back(DownloadItem{c->d.curv, 0, 1, 1, curv});
+    HIPCHK(c, c->dl.run(L, c->stream, items));
     return MFLBM_OK;
 }
 

@@ -20,6 +20,7 @@
 
 #include "batch_plan.h"
 #include "device_common.h"
+#include "download.h"
 #include "lattice.h"
 #include "mflbm.h"
 #include "sp_kernels.h"
@@ -193,6 +194,7 @@ struct mflbm_spb_ctx {
     int* nactive_h = nullptr;            // pinned
     double* staging = nullptr;           // dense upload/download buffer (19 arrays of the largest sample)
     long staging_len = 0;
+    Downloader dl;                       // pinned ring of the downloads
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     bool committed = false;
@@ -394,6 +396,7 @@ extern "C" void mflbm_spb_destroy(mflbm_spb_ctx* c) {
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     free_all(c);
+    c->dl.free();
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -622,13 +625,10 @@ extern "C" int mflbm_spb_download_state(mflbm_spb_ctx* c, int32_t sample, double
                c->p.rest_state ? rest_weight(q) : lat::W[q]);
     rc = c->fp32 ? scatter_sample<float>(c, sample) : scatter_sample<double>(c, sample);
     if (rc) return rc;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    std::vector<double> buf(L.total);
-    for (int q = 0; q < 19; ++q) {
-        if (!f[q]) continue;
-        HIPCHK(c, hipMemcpy(buf.data(), c->staging + q * L.total, sizeof(double) * L.total, hipMemcpyDeviceToHost));
-        unpack_host(L, 1, buf.data(), f[q]);
-    }
+    std::vector<DownloadItem> items;
+    for (int q = 0; q < 19; ++q)
+        if (f[q]) items.push_back(DownloadItem{c->staging + q * L.total, 0, 1, 1, f[q]});
+    HIPCHK(c, c->dl.run(L, c->stream, items));
     return MFLBM_OK;
 }
 
@@ -651,14 +651,11 @@ extern "C" int mflbm_spb_download_macro(mflbm_spb_ctx* c, int32_t sample, double
         const SDev<double>& d = c->dev64[sample];
         LAUNCH(c, k_sp_macro<double>, nblocks(d.nf), d, c->p.force_z, st, st + ps, st + 2 * ps, st + 3 * ps);
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    std::vector<double> buf(L.total);
     double* dst[4] = {u, v, w, rho};
-    for (int m = 0; m < 4; ++m) {
-        if (!dst[m]) continue;
-        HIPCHK(c, hipMemcpy(buf.data(), st + m * ps, sizeof(double) * L.total, hipMemcpyDeviceToHost));
-        unpack_host(L, 1, buf.data(), dst[m]);
-    }
+    std::vector<DownloadItem> items;
+    for (int m = 0; m < 4; ++m)
+        if (dst[m]) items.push_back(DownloadItem{st + m * ps, 0, 1, 1, dst[m]});
+    HIPCHK(c, c->dl.run(L, c->stream, items));
     return MFLBM_OK;
 }
 

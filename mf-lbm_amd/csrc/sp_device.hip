@@ -19,6 +19,7 @@
 
 #include "collide_sp.h"
 #include "device_common.h"
+#include "download.h"
 #include "lattice.h"
 #include "mflbm.h"
 #include "sp_kernels.h"
@@ -275,6 +276,7 @@ struct mflbm_sp_ctx {
     int8_t* walls = nullptr;
     double* planes = nullptr;    // w_in, cf (19)
     double* red = nullptr;       // monitor layer results (3*nz)
+    Downloader dl;               // pinned ring of the downloads
     void* compact = nullptr;     // 19 population slices (compact slots + link slots), double or float
     int* map = nullptr;
     RowRec* rows = nullptr;
@@ -502,6 +504,7 @@ extern "C" void mflbm_sp_destroy(mflbm_sp_ctx* c) {
     for (auto e : c->ev)
         if (e) (void)hipEventDestroy(e);
     sp_free_geometry(c);
+    c->dl.free();
     void* bufs[] = {c->dense_pdf, c->fields, c->walls, c->planes, c->red};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
@@ -691,13 +694,10 @@ extern "C" int mflbm_sp_download_state(mflbm_sp_ctx* c, double* const* f, double
     const Layout& L = c->L;
     const int rc = c->fp32 ? sp_scatter_t<float>(c) : sp_scatter_t<double>(c);
     if (rc) return rc;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    std::vector<double> buf(L.total);
-    for (int q = 0; q < 19 && f; ++q) {
-        if (!f[q]) continue;
-        HIPCHK(c, hipMemcpy(buf.data(), c->dense_pdf + q * c->ps, sizeof(double) * L.total, hipMemcpyDeviceToHost));
-        unpack_host(L, 1, buf.data(), f[q]);
-    }
+    std::vector<DownloadItem> items;
+    for (int q = 0; q < 19 && f; ++q)
+        if (f[q]) items.push_back(DownloadItem{c->dense_pdf + q * c->ps, 0, 1, 1, f[q]});
+    HIPCHK(c, c->dl.run(L, c->stream, items));
     const size_t plane = (size_t)(L.nx + 2) * (L.ny + 2);
     if (f_convec) HIPCHK(c, hipMemcpy(f_convec, c->d.cf, sizeof(double) * plane * 19, hipMemcpyDeviceToHost));
     return MFLBM_OK;
@@ -750,14 +750,11 @@ extern "C" int mflbm_sp_monitor(mflbm_sp_ctx* c, double* layers, double* umax2) 
 extern "C" int mflbm_sp_download_macro(mflbm_sp_ctx* c, double* u, double* v, double* w, double* rho) {
     if (!c) return MFLBM_ERR_ARG;
     const Layout& L = c->L;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    std::vector<double> buf(L.total);
     double* dst[4] = {u, v, w, rho};
-    for (int m = 0; m < 4; ++m) {
-        if (!dst[m]) continue;
-        HIPCHK(c, hipMemcpy(buf.data(), c->fields + m * c->ps, sizeof(double) * L.total, hipMemcpyDeviceToHost));
-        unpack_host(L, 1, buf.data(), dst[m]);
-    }
+    std::vector<DownloadItem> items;
+    for (int m = 0; m < 4; ++m)
+        if (dst[m]) items.push_back(DownloadItem{c->fields + m * c->ps, 0, 1, 1, dst[m]});
+    HIPCHK(c, c->dl.run(L, c->stream, items));
     return MFLBM_OK;
 }
 
