@@ -21,6 +21,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int NT = 256;
+constexpr int NXCD = 8;   // gfx950: 8 dies, work-groups dispatched to them in turn
 
 __device__ __forceinline__ float bf2f(__bf16 v) { return (float)v; }
 __device__ __forceinline__ __bf16 f2bf(float v) { return (__bf16)v; }
@@ -125,118 +126,197 @@ __global__ void __launch_bounds__(NT) k_conv_fwd(const __bf16* __restrict__ x, c
 
 // Weight gradient: dw[co][k] += sum_p dy[p][co] * x[p + off(k)][ci(k)] (rows of 27 cin, the layout of the FP32
 // master weights), the positions split into chunks of `chunk` (a multiple of 32) over grid z.  A work-group computes
-// 32 output channels x 128 k (one wave per 32 k) and walks its chunk 32 positions at a time: the dy tile (32
-// positions x 32 channels) and the im2col tile of x (32 positions x 128 k) are loaded with 16-byte accesses (8
-// channels of one position) and stored transposed in LDS, two buffers in turn (the next tile's loads are in flight
-// while the current one is multiplied), and each wave reads its fragments from there.  The fragments, and so the
-// sums, are those of a lane-by-lane gather: lane l takes 8 consecutive positions for one channel (A) or one k (B).
+// 16 NC output channels x 16 input channels x all 27 offsets and walks its chunk 32 positions at a time; wave v takes
+// the offsets 7 v .. 7 v + 6, so one dy fragment serves seven products.  w is a multiple of 8, so eight positions from
+// a multiple of 8 on lie in one x row: per such octet and per (dz, dy) the rows x - 1 .. x + 8 are staged (zero outside
+// the domain), and an offset's operand is those rows from dx on.  Both tiles are staged as they lie in memory,
+// [position][channel], 16 bytes at a time, two buffers in turn, and the transposing LDS read of gfx950 hands each lane
+// the positions of its channel (of 16 lanes, lane 4 j + c / 4 addresses row j, channels 4 (c / 4) .., and lane c receives
+// rows 0 .. 3 of channel c).  The fragments, and so the sums, are those of a lane-by-lane gather: lane l takes the
+// 8 consecutive positions from 8 (l / 16) on of one output channel (A) or one input channel (B).
+// Bound by the latency of a tile (load, barrier, LDS reads, 7 NC products) with few waves on each compute unit: the
+// chunk fixes the order of the sums, so a work-group walks all 128 tiles.  4 x 32^3, 64 -> 64, with the chunk sums: 567
+// us with scalar transposing stores, 88 us so; 4 x 64^3, 32 -> 32: 1010 and 154 us (377 TFLOP/s).
 // The chunk sums go to dw with FP32 atomics, or (ORDERED) are stored to the chunk's own slice dw + z * cout * K,
 // every element written by exactly one lane, for a fixed-order sum after.
-constexpr int DW_KT = 128;          // k per work-group
-constexpr int DW_LD = 40;           // LDS row length (32 positions + 8: 80-byte rows keep 16-byte fragment reads aligned)
-template <bool ORDERED>
-__global__ void __launch_bounds__(NT) k_conv_dw(const __bf16* __restrict__ x, const __bf16* __restrict__ dy,
-                                                float* __restrict__ dw, Shape S, int cin, int cout, long chunk) {
-    __shared__ __attribute__((aligned(16))) __bf16 As[2][32][DW_LD];
-    __shared__ __attribute__((aligned(16))) __bf16 Bs[2][DW_KT][DW_LD];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ bf16x8 read_transposed(const __bf16* lo, const __bf16* hi) {
+    union {
+        s16x4 h[2];
+        bf16x8 v;
+    } u;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)lo);
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)hi);
+    return u.v;
+}
+// Global reads go through a buffer resource over the chunk and its neighbours: an item outside the domain or the layer
+// takes an offset beyond it and reads zero, so no load sits under a branch (it would have to arrive before the branch
+// is left) and nothing is cleared on the way to LDS.  Wave v stages octet v of the tile, whose coordinates are scalar;
+// each item needs some of seven conditions on them (a lane constant).  FAR: the window is 2 GiB or more (planes of
+// hundreds of millions of values); the same loads by 64-bit addresses.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+constexpr int DW_OFF = 7;    // offsets per wave
+constexpr int DW_ROWS = 9 * 4 * 10;   // staged x rows of a tile: (dz, dy) x octet x (x - 1 .. x + 8)
+constexpr unsigned NOWHERE = 1u << 31;
+__host__ __device__ inline long dw_window(const Shape& S, int cin, long chunk) {   // bytes of x a chunk may touch
+    return (chunk + 8 + 2 * ((long)S.h * S.w + S.w + 1)) * cin * 2;
+}
+template <bool ORDERED, int NC, bool FAR>
+__global__ void __launch_bounds__(NT, 2) k_conv_dw(const __bf16* __restrict__ x, const __bf16* __restrict__ dy,
+                                                   float* __restrict__ dw, Shape S, int cin, int cout, long chunk,
+                                                   int nco, int nci, int total) {
+    __shared__ __attribute__((aligned(16))) __bf16 xs[2][DW_ROWS][16];
+    __shared__ __attribute__((aligned(16))) __bf16 ys[2][NC][32][16];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, q = lane >> 4;
-    const int co0 = blockIdx.x * 32;
-    const int kb0 = blockIdx.y * DW_KT;
+    // each die takes a run of consecutive chunks, all channel groups of one next to each other: they share its L2
+    const int g = (int)(blockIdx.x % NXCD) * (int)(gridDim.x / NXCD) + (int)(blockIdx.x / NXCD);
+    if (g >= total) return;
+    const int zc = g / (nco * nci);
+    const int co0 = (g % nco) * (16 * NC);
+    const int ci0 = (g / nco % nci) * 16;
     const int K = 27 * cin;
     const long M = S.count();
-    const long pbeg = (long)blockIdx.z * chunk;
-    const long pend = pbeg + chunk < M ? pbeg + chunk : M;
-    const int ntile = (int)((pend - pbeg + 31) / 32);
-    const bf16x8 zero = {};
-    // this thread's loads of a tile: one dy chunk (threads < 128: position tid / 4, channels 8 (tid % 4) ..) and two
-    // x chunks (item u = tid + 256 v: position u / 16, k 8 (u % 16) .. of the work-group's 128)
-    auto load = [&](long pk, bf16x8& ra, bf16x8 (&rb)[2]) {
-        ra = zero;
-        if (tid < 128) {
-            const long p = pk + (tid >> 2);
-            const int co = co0 + 8 * (tid & 3);
-            if (p < pend && co < cout) ra = *(const bf16x8*)(dy + p * cout + co);
-        }
+    const long pbeg = (long)zc * chunk;
+    const int npos = (int)((pbeg + chunk < M ? pbeg + chunk : M) - pbeg);
+    const int ntile = (npos + 31) / 32;
+    // the x window: position pbeg - lead is its start (before x's own start only where no item is valid)
+    const long lead = (long)S.h * S.w + S.w + 1;
+    const __bf16* const xwin = x + (pbeg - lead) * cin;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)xwin, 0, FAR ? 0 : (int)dw_window(S, cin, chunk), 0x00027000);
+    const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc((void*)(dy + pbeg * cout), 0, FAR ? 0 : npos * cout * 2, 0x00027000);
+    // this lane's x items of octet wv: item u = lane + 64 v: channels 8 (u % 2) .. of row u / 2 = (dz, dy) x (x - 1 .. x + 8)
+    constexpr int NX = 3;
+    unsigned req[NX], xo[NX];
+    long xl[NX];
+    int xrow[NX];
 #pragma unroll
-        for (int v = 0; v < 2; ++v) {
-            const int u = tid + NT * v;
-            const long p = pk + (u >> 4);
-            const int k = kb0 + 8 * (u & 15);
-            rb[v] = zero;
-            if (p < pend && k < K) {
-                const int off = k / cin, ci = k - off * cin;
-                int t = (int)p;   // (positions are below 2^31: 32-bit decode)
-                const int xq = t % S.w;
-                t /= S.w;
-                const int yq = t % S.h;
-                t /= S.h;
-                const int zq = t % S.d;
-                const int nq = t / S.d;
-                const int zz = zq + off / 9 - 1, yy = yq + (off / 3) % 3 - 1, xx = xq + off % 3 - 1;
-                if (zz >= 0 && zz < S.d && yy >= 0 && yy < S.h && xx >= 0 && xx < S.w)
-                    rb[v] = *(const bf16x8*)(x + ((((long)nq * S.d + zz) * S.h + yy) * S.w + xx) * cin + ci);
-            }
-        }
-    };
-    auto store = [&](int buf, const bf16x8& ra, const bf16x8 (&rb)[2]) {
-        if (tid < 128) {
-            const int pl = tid >> 2, c = 8 * (tid & 3);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) As[buf][c + j][pl] = ra[j];
-        }
-#pragma unroll
-        for (int v = 0; v < 2; ++v) {
-            const int u = tid + NT * v;
-            const int pl = u >> 4, kl = 8 * (u & 15);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) Bs[buf][kl + j][pl] = rb[v][j];
-        }
-    };
-    f32x4 acc[2][2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int g = 0; g < 2; ++g) acc[h][g] = f32x4{0.f, 0.f, 0.f, 0.f};
-    bf16x8 ra, rb[2];
-    if (ntile > 0) {
-        load(pbeg, ra, rb);
-        store(0, ra, rb);
+    for (int v = 0; v < NX; ++v) {
+        const int u = lane + 64 * v, row = u >> 1, e = row / 10, c = row % 10;
+        const int dz = e / 3 - 1, dyy = e % 3 - 1, ci = ci0 + 8 * (u & 1);
+        // conditions on the octet: 0 y > 0, 1 y < h - 1, 2 z > 0, 3 z < d - 1, 4 x > 0, 5 x + 8 < w, 6 in the chunk, 7 never
+        req[v] = (dyy < 0 ? 1u : dyy > 0 ? 2u : 0u) | (dz < 0 ? 4u : dz > 0 ? 8u : 0u) | (c == 0 ? 16u : c == 9 ? 32u : 0u) |
+                 64u | (u < 180 && ci < cin ? 0u : 128u);
+        xl[v] = (lead + 8 * wv + ((long)dz * S.h + dyy) * S.w + c - 1) * cin + ci;   // elements from the window's start
+        xo[v] = (unsigned)(2 * xl[v]);
+        xrow[v] = min(e, 8) * 40 + wv * 10 + c;
     }
-    __syncthreads();
-    for (int it = 0; it < ntile; ++it) {
-        const int buf = it & 1;
-        const bool more = it + 1 < ntile;
-        if (more) load(pbeg + 32L * (it + 1), ra, rb);
-        bf16x8 fa[2], fb[2];
+    int ox, oy, oz;   // the octet's coordinates
+    {
+        int t = (int)(pbeg + 8 * wv);   // (positions are below 2^31: 32-bit decode)
+        ox = t % S.w;
+        t /= S.w;
+        oy = t % S.h;
+        t /= S.h;
+        oz = t % S.d;
+    }
+    const int ax = 32 % S.w, ay = (32 / S.w) % S.h, az = (32 / S.w) / S.h % S.d;   // 32 positions on: one carry an axis
+    const int yc = tid % (2 * NC), yp = tid / (2 * NC);   // dy item: channels 8 yc .. of position yp
+    const bool yact = tid < 64 * NC;
+    const unsigned yo = yact && co0 + 8 * yc < cout ? 2u * (unsigned)(yp * cout + co0 + 8 * yc) : NOWHERE;
+    auto load = [&](int it, u32x4& ra, u32x4 (&rb)[NX]) {
+        const unsigned have = (oy > 0 ? 1u : 0u) | (oy < S.h - 1 ? 2u : 0u) | (oz > 0 ? 4u : 0u) | (oz < S.d - 1 ? 8u : 0u) |
+                              (ox > 0 ? 16u : 0u) | (ox + 8 < S.w ? 32u : 0u) | (32 * it + 8 * wv < npos ? 64u : 0u);
+        if constexpr (FAR) {
+            const u32x4 none = {};
+            ra = yo != NOWHERE && 32 * it + yp < npos
+                     ? *(const u32x4*)(dy + (pbeg + 32L * it + yp) * cout + co0 + 8 * yc) : none;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) fa[h] = *(const bf16x8*)&As[buf][h * 16 + r][q * 8];
+            for (int v = 0; v < NX; ++v) rb[v] = (req[v] & ~have) == 0 ? *(const u32x4*)(xwin + xl[v] + 32L * it * cin) : none;
+        } else {
+            ra = __builtin_amdgcn_raw_buffer_load_b128(yr, (int)(32 * it + yp < npos ? yo : NOWHERE), 64 * it * cout, 0);
 #pragma unroll
-        for (int g = 0; g < 2; ++g) fb[g] = *(const bf16x8*)&Bs[buf][wv * 32 + g * 16 + r][q * 8];
+            for (int v = 0; v < NX; ++v)
+                rb[v] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)((req[v] & ~have) == 0 ? xo[v] : NOWHERE), 64 * it * cin, 0);
+        }
+        ox += ax;
+        const int cx = ox >= S.w;
+        ox -= cx ? S.w : 0;
+        oy += ay + cx;
+        const int cy = oy >= S.h;
+        oy -= cy ? S.h : 0;
+        oz += az + cy;
+        oz -= oz >= S.d ? S.d : 0;
+    };
+    auto store = [&](int buf, const u32x4& ra, const u32x4 (&rb)[NX]) {
+        if (yact) *(u32x4*)&ys[buf][yc >> 1][yp][8 * (yc & 1)] = ra;
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int v = 0; v < NX; ++v)
+            if (lane + 64 * v < 180) *(u32x4*)&xs[buf][xrow[v]][8 * (lane & 1)] = rb[v];
+    };
+    f32x4 acc[NC][DW_OFF];
 #pragma unroll
-            for (int g = 0; g < 2; ++g) acc[h][g] = mfma(fa[h], fb[g], acc[h][g]);
-        if (more) store(buf ^ 1, ra, rb);
+    for (int h = 0; h < NC; ++h)
+#pragma unroll
+        for (int o = 0; o < DW_OFF; ++o) acc[h][o] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int tr = r >> 2, tc = 4 * (r & 3);   // row and first channel this lane addresses in a transposing read
+    int row[DW_OFF];
+#pragma unroll
+    for (int o = 0; o < DW_OFF; ++o) {
+        const int off = min(wv * DW_OFF + o, 26);   // (the last wave's seventh is computed twice and not stored)
+        row[o] = (off / 3) * 40 + off % 3 + 10 * q + tr;
+    }
+    // tile `it` is in buffer it % 2; its successor is already in one set of registers, and the loads of the one after
+    // that go to the other set, so a load has two tiles of products to arrive
+    u32x4 ra[2], rb[2][NX];
+    auto step = [&](int it, int cur) {
+        if (it + 2 < ntile) load(it + 2, ra[cur], rb[cur]);
+        bf16x8 fa[NC], fb[DW_OFF];
+#pragma unroll
+        for (int h = 0; h < NC; ++h) fa[h] = read_transposed(&ys[cur][h][8 * q + tr][tc], &ys[cur][h][8 * q + 4 + tr][tc]);
+#pragma unroll
+        for (int o = 0; o < DW_OFF; ++o) fb[o] = read_transposed(&xs[cur][row[o]][tc], &xs[cur][row[o] + 4][tc]);
+#pragma unroll
+        for (int o = 0; o < DW_OFF; ++o)
+#pragma unroll
+            for (int h = 0; h < NC; ++h) acc[h][o] = mfma(fa[h], fb[o], acc[h][o]);
+        if (it + 1 < ntile) store(cur ^ 1, ra[cur ^ 1], rb[cur ^ 1]);
         __syncthreads();
+    };
+    if (ntile > 0) load(0, ra[0], rb[0]);
+    if (ntile > 1) load(1, ra[1], rb[1]);
+    if (ntile > 0) store(0, ra[0], rb[0]);
+    __syncthreads();
+    int it = 0;
+    for (; it + 1 < ntile; it += 2) {
+        step(it, 0);
+        step(it + 1, 1);
     }
-    const int kk0 = kb0 + wv * 32;
+    if (it < ntile) step(it, 0);
+    const int ci = ci0 + r;
+    if (ci >= cin) return;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int o = 0; o < DW_OFF; ++o) {
+        const int off = wv * DW_OFF + o;
+        if (off >= 27) continue;
+        const int kcol = off * cin + ci;
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const int kcol = kk0 + g * 16 + r;
-            if (kcol >= K) continue;
+        for (int h = 0; h < NC; ++h)
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const int co = co0 + h * 16 + q * 4 + t;
                 if (co >= cout) continue;
                 if (ORDERED)
-                    dw[((long)blockIdx.z * cout + co) * K + kcol] = acc[h][g][t];
+                    dw[((long)zc * cout + co) * K + kcol] = acc[h][o][t];
                 else
-                    atomicAdd(&dw[(long)co * K + kcol], acc[h][g][t]);
+                    atomicAdd(&dw[(long)co * K + kcol], acc[h][o][t]);
             }
-        }
+    }
+}
+// Output channels per work-group: 32 (fewer fragment reads per product) where that leaves a work-group for each of the
+// 256 compute units, else 16.  Measured, 32 against 16: 4 x 32^3 64 -> 64 (256 work-groups of 32) 88 / 101 us, 4 x 16^3
+// 256 -> 128 (256) 83 / 86, 4 x 64^3 32 -> 32 (512) 154 / 188; 4 x 32^3 32 -> 64 (128) 76 / 70, 4 x 16^3 128 -> 128
+// (128) 70 / 64, 4 x 8^3 256 -> 256 (128) 44 / 41.  (64 channels: within 2 % at best, 190 at 4 x 64^3 32 -> 32.)
+template <bool ORDERED>
+void launch_conv_dw(const void* x, const void* dy, float* dw, const Shape& S, int cin, int cout, long chunk, hipStream_t st) {
+    const long nz = (S.count() + chunk - 1) / chunk, ny = (cin + 15) / 16;
+    const int nc = cout > 16 && (cout + 31) / 32 * ny * nz >= 256 ? 2 : 1;
+    const bool far = dw_window(S, cin, chunk) >= (1L << 31) || chunk * cout * 2 >= (1L << 31);
+    const auto kern = far ? k_conv_dw<ORDERED, 1, true> : nc == 2 ? k_conv_dw<ORDERED, 2, false> : k_conv_dw<ORDERED, 1, false>;
+    const int nco = (cout + 16 * (far ? 1 : nc) - 1) / (16 * (far ? 1 : nc));
+    const long total = nco * ny * nz;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((total + NXCD - 1) / NXCD * NXCD)), dim3(NT), 0, st, (const __bf16*)x,
+                       (const __bf16*)dy, dw, S, cin, cout, chunk, nco, (int)ny, (int)total);
 }
 
 // positions per chunk of the weight- and bias-gradient sums
@@ -419,9 +499,7 @@ extern "C" int mflbm_nn_conv3d_dw(const void* x, const void* dy, float* dw, floa
         return MFLBM_ERR_ARG;
     const Shape S{n, d, h, w};
     const long M = S.count();
-    const dim3 grid((unsigned)((cout + 31) / 32), (unsigned)((27 * cin + 127) / 128), (unsigned)((M + DW_CHUNK - 1) / DW_CHUNK));
-    hipLaunchKernelGGL(k_conv_dw<false>, grid, dim3(NT), 0, (hipStream_t)stream, (const __bf16*)x, (const __bf16*)dy, dw,
-                       S, (int)cin, (int)cout, DW_CHUNK);
+    launch_conv_dw<false>(x, dy, dw, S, cin, cout, DW_CHUNK, (hipStream_t)stream);
     if (dbias)
         hipLaunchKernelGGL(k_bias_grad<false>, dim3((unsigned)((M + DB_CHUNK - 1) / DB_CHUNK), (unsigned)((cout + 31) / 32)),
                            dim3(NT), 0, (hipStream_t)stream, (const __bf16*)dy, dbias, M, (int)cout, DB_CHUNK);
@@ -444,9 +522,7 @@ int dw_ordered_launch(const void* x, const void* dy, float* dw, float* dbias, fl
     const long M = S.count();
     const long K = 27L * cin, nzw = (M + DW_CHUNK - 1) / DW_CHUNK, nzb = (M + DB_CHUNK - 1) / DB_CHUNK;
     float* bpart = work + nzw * cout * K;
-    const dim3 grid((unsigned)((cout + 31) / 32), (unsigned)((K + 127) / 128), (unsigned)nzw);
-    hipLaunchKernelGGL(k_conv_dw<true>, grid, dim3(NT), 0, st, (const __bf16*)x, (const __bf16*)dy, work, S, (int)cin,
-                       (int)cout, DW_CHUNK);
+    launch_conv_dw<true>(x, dy, work, S, cin, cout, DW_CHUNK, st);
     hipLaunchKernelGGL(k_sum_slices, dim3((unsigned)((cout * K + NT - 1) / NT)), dim3(NT), 0, st, (const float*)work, dw,
                        cout * K, (int)nzw);
     if (dbias) {
