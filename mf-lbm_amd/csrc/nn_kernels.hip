@@ -18,9 +18,12 @@
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int NT = 256;
+constexpr unsigned NOWHERE = 1u << 31;   // a byte offset beyond every buffer resource: such a load reads zero
 constexpr int NXCD = 8;   // gfx950: 8 dies, work-groups dispatched to them in turn
 
 __device__ __forceinline__ float bf2f(__bf16 v) { return (float)v; }
@@ -124,6 +127,190 @@ __global__ void __launch_bounds__(NT) k_conv_fwd(const __bf16* __restrict__ x, c
         }
 }
 
+// The same convolution from a spatial tile in LDS: a work-group owns TZ x TY x TX positions and 16 NCO WC output
+// channels, stages the tile's input with its one-node halo once (all cin channels; zero outside the domain) and takes all
+// 27 offsets from there, so each input value is read from memory about 2.3 times instead of 27.  Wave (wp, wc) computes
+// 16 MT positions x 16 NCO channels; the weights of KG steps of 32 k come through LDS in fragment order (16 bytes per
+// lane, linear), two buffers in turn, the next stage's loads in flight.  Rows of the input tile are an odd number of
+// 16-byte chunks apart, so the 16 positions of a fragment fall on different banks.  The k order, and so every sum, is
+// that of k_conv_fwd; weights are the A operand, so a lane ends with four consecutive channels of one position.
+template <int MT, int NCO, int WP, int WC, int TZ, int TY, int TX, int KG>
+struct ConvTile {
+    static constexpr int THREADS = 64 * WP * WC, POS = TZ * TY * TX, CO = 16 * NCO * WC;
+    static constexpr int HX = TX + 2, HY = TY + 2, HZ = TZ + 2, ROWS = HX * HY * HZ;
+    static constexpr int WITEMS = KG * CO * 4;   // 16-byte chunks of a weight stage
+    static_assert(POS == 16 * MT * WP && WITEMS % THREADS == 0, "tile split");
+    static int lds_bytes(int cin) { return ((ROWS * ((cin / 8) | 1) + 1) + 2 * WITEMS) * 16; }
+};
+template <int RELU, bool UNI, int MT, int NCO, int WP, int WC, int TZ, int TY, int TX, int KG>
+__global__ void __launch_bounds__(64 * WP * WC) k_conv_tile(const __bf16* __restrict__ x, const __bf16* __restrict__ wt,
+                                                            const float* __restrict__ bias, __bf16* __restrict__ y, Shape S,
+                                                            int cin, int cout, int kpad, int nxt, int nyt, int nzt, int ncg,
+                                                            int total) {
+    using T = ConvTile<MT, NCO, WP, WC, TZ, TY, TX, KG>;
+    extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
+    const int g0 = (int)(blockIdx.x % NXCD) * (int)(gridDim.x / NXCD) + (int)(blockIdx.x / NXCD);   // a die: consecutive tiles
+    if (g0 >= total) return;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wp = wv % WP, wc = wv / WP;
+    const int r = lane & 15, q = lane >> 4;
+    int t = g0;
+    const int co0 = (t % ncg) * T::CO;
+    t /= ncg;
+    const int x0 = (t % nxt) * TX;
+    t /= nxt;
+    const int y0 = (t % nyt) * TY;
+    t /= nyt;
+    const int z0 = (t % nzt) * TZ;
+    const int nn = t / nzt;
+    const int nch = cin / 8, sc = nch | 1;
+    u32x4* const xs = lds;                              // ROWS rows of sc chunks, then a zero chunk
+    u32x4* const ws = lds + T::ROWS * sc + 1;           // two stages of weight fragments
+    const u32x4 none = {};
+    // input tile through a buffer resource over its planes (the launcher keeps the window below 2 GiB); an item outside
+    // the domain takes an offset beyond it and reads zero
+    const long plane = (long)S.h * S.w;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(x + ((long)nn * S.d + z0 - 1) * plane * cin), 0, (int)(T::HZ * plane * cin * 2), 0x00027000);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)wt, 0, cout * kpad * 2, 0x00027000);
+    const int nk = kpad / 32, ns = (nk + KG - 1) / KG;
+    // weight items: chunk q of step kk of channel c: 64 KG contiguous bytes of a channel's row per 4 KG threads
+    constexpr int NW = T::WITEMS / T::THREADS;
+    unsigned wo[NW];
+    int wl[NW];
+#pragma unroll
+    for (int v = 0; v < NW; ++v) {
+        const int u = tid + T::THREADS * v, uq = u & 3, kk = (u >> 2) % KG, c = (u >> 2) / KG;
+        wo[v] = co0 + c < cout ? 2u * (unsigned)((co0 + c) * kpad + kk * 32 + uq * 8) : NOWHERE;
+        wl[v] = ((kk * (T::CO / 16) + (c >> 4)) * 4 + uq) * 16 + (c & 15);
+    }
+    u32x4 rw[NW];
+    auto wload = [&](int s) {
+#pragma unroll
+        for (int v = 0; v < NW; ++v) {
+            const int kk = ((tid + T::THREADS * v) >> 2) % KG;   // (a step past the row's end is not read)
+            rw[v] = __builtin_amdgcn_raw_buffer_load_b128(wr, (int)(s * KG + kk < nk ? wo[v] : NOWHERE), s * KG * 64, 0);
+        }
+    };
+    auto wstore = [&](int buf) {
+#pragma unroll
+        for (int v = 0; v < NW; ++v) ws[buf * T::WITEMS + wl[v]] = rw[v];
+    };
+    wload(0);
+    {
+        const int items = T::ROWS * nch;
+        constexpr int UN = 8;   // loads in flight per thread
+        for (int u0 = tid; u0 < items; u0 += UN * T::THREADS) {
+            u32x4 v[UN];
+            int at[UN];
+#pragma unroll
+            for (int k = 0; k < UN; ++k) {
+                const int u = u0 + k * T::THREADS;
+                const int row = u / nch, c = u - row * nch;
+                const int hx = row % T::HX, hy = (row / T::HX) % T::HY, hz = row / (T::HX * T::HY);
+                const int zz = z0 - 1 + hz, yy = y0 - 1 + hy, xx = x0 - 1 + hx;
+                const bool in = (u < items) & ((unsigned)zz < (unsigned)S.d) & ((unsigned)yy < (unsigned)S.h) & ((unsigned)xx < (unsigned)S.w);
+                at[k] = row * sc + c;
+                v[k] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(in ? (((unsigned)hz * S.h + yy) * S.w + xx) * (unsigned)cin * 2u + 16u * c : NOWHERE), 0, 0);
+            }
+#pragma unroll
+            for (int k = 0; k < UN; ++k)
+                if (u0 + k * T::THREADS < items) xs[at[k]] = v[k];
+        }
+        if (tid == 0) xs[T::ROWS * sc] = none;
+    }
+    wstore(0);
+    // first chunk of the row of this lane's position in each fragment
+    int rb[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int p = (wp * MT + m) * 16 + r;
+        rb[m] = ((p / (TX * TY) * T::HY + p / TX % TY) * T::HX + p % TX) * sc;
+    }
+    f32x4 acc[MT][NCO];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int c = 0; c < NCO; ++c) acc[m][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // One step of 32 k: this lane's eight k are one channel chunk of one offset; with cin a multiple of 32 (UNI) the
+    // offset is the whole wave's, else the division goes by a multiplication (k8 / nch = k8 * inv >> 16 for k8 < 65536 /
+    // nch) and the last step may reach beyond the 27 offsets (zero chunk).
+    const unsigned inv = (65536u + nch - 1) / nch;
+    auto products = [&](const u32x4* w, int ks) {
+        const unsigned k8 = UNI ? (unsigned)ks * 4u : (unsigned)(ks * 4 + q);
+        const unsigned off = k8 * inv >> 16, c8 = k8 - off * nch + (UNI ? q : 0);
+        const unsigned dz = off * 57u >> 9, e = off - 9u * dz, dyy = e * 11u >> 5;
+        const int ko = (int)(((dz * T::HY + dyy) * T::HX + (e - 3u * dyy)) * (unsigned)sc + c8);
+        bf16x8 fw[NCO], fx[MT];
+#pragma unroll
+        for (int c = 0; c < NCO; ++c) fw[c] = __builtin_bit_cast(bf16x8, w[c * 64]);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) fx[m] = __builtin_bit_cast(bf16x8, xs[UNI || off < 27u ? rb[m] + ko : T::ROWS * sc]);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int c = 0; c < NCO; ++c) acc[m][c] = mfma(fw[c], fx[m], acc[m][c]);
+    };
+    __syncthreads();
+    for (int s = 0; s < ns; ++s) {
+        if (s + 1 < ns) wload(s + 1);
+        const u32x4* const w = ws + (s & 1) * T::WITEMS + wc * NCO * 64 + lane;
+        if ((s + 1) * KG <= nk) {   // (whole stages without a branch between their products)
+#pragma unroll
+            for (int kk = 0; kk < KG; ++kk) products(w + kk * T::CO * 4, s * KG + kk);
+        } else {
+            for (int kk = 0; s * KG + kk < nk; ++kk) products(w + kk * T::CO * 4, s * KG + kk);
+        }
+        if (s + 1 < ns) wstore((s + 1) & 1);
+        __syncthreads();
+    }
+    const bool quad = cout % 4 == 0 && ((uintptr_t)y & 7) == 0;
+#pragma unroll
+    for (int c = 0; c < NCO; ++c) {
+        const int co = co0 + (wc * NCO + c) * 16 + 4 * q;
+        float bb[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) bb[k] = bias && co + k < cout ? bias[co + k] : 0.f;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int p = (wp * MT + m) * 16 + r;
+            const int zz = z0 + p / (TX * TY), yy = y0 + p / TX % TY, xx = x0 + p % TX;
+            if (zz >= S.d || yy >= S.h || xx >= S.w) continue;
+            __bf16* const out = y + (((long)nn * S.d + zz) * plane + (long)yy * S.w + xx) * cout + co;
+            bf16x4 o;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float v = acc[m][c][k] + bb[k];
+                if (RELU && v < 0.f) v = 0.f;
+                o[k] = f2bf(v);
+            }
+            if (quad) {
+                if (co < cout) *(bf16x4*)out = o;
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (co + k < cout) out[k] = o[k];
+            }
+        }
+    }
+}
+template <int MT, int NCO, int WP, int WC, int TZ, int TY, int TX, int KG>
+int launch_conv_tile(const void* x, const void* wf, const float* bias, void* y, const Shape& S, int cin, int cout, int kpad,
+                     int relu, hipStream_t st) {
+    using T = ConvTile<MT, NCO, WP, WC, TZ, TY, TX, KG>;
+    const int nxt = (S.w + TX - 1) / TX, nyt = (S.h + TY - 1) / TY, nzt = (S.d + TZ - 1) / TZ, ncg = (cout + T::CO - 1) / T::CO;
+    const long total = (long)nxt * nyt * nzt * S.n * ncg;
+    const int bytes = T::lds_bytes(cin);
+    const bool uni = cin % 32 == 0;
+    const auto kern = relu ? (uni ? k_conv_tile<1, true, MT, NCO, WP, WC, TZ, TY, TX, KG> : k_conv_tile<1, false, MT, NCO, WP, WC, TZ, TY, TX, KG>)
+                           : (uni ? k_conv_tile<0, true, MT, NCO, WP, WC, TZ, TY, TX, KG> : k_conv_tile<0, false, MT, NCO, WP, WC, TZ, TY, TX, KG>);
+    if (bytes > 65536 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)
+        return MFLBM_ERR_HIP;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((total + NXCD - 1) / NXCD * NXCD)), dim3(T::THREADS), bytes, st, (const __bf16*)x,
+                       (const __bf16*)wf, bias, (__bf16*)y, S, cin, cout, kpad, nxt, nyt, nzt, ncg, (int)total);
+    return hipGetLastError() == hipSuccess ? MFLBM_OK : MFLBM_ERR_HIP;
+}
+
 // Weight gradient: dw[co][k] += sum_p dy[p][co] * x[p + off(k)][ci(k)] (rows of 27 cin, the layout of the FP32
 // master weights), the positions split into chunks of `chunk` (a multiple of 32) over grid z.  A work-group computes
 // 16 NC output channels x 16 input channels x all 27 offsets and walks its chunk 32 positions at a time; wave v takes
@@ -154,10 +341,8 @@ __device__ __forceinline__ bf16x8 read_transposed(const __bf16* lo, const __bf16
 // is left) and nothing is cleared on the way to LDS.  Wave v stages octet v of the tile, whose coordinates are scalar;
 // each item needs some of seven conditions on them (a lane constant).  FAR: the window is 2 GiB or more (planes of
 // hundreds of millions of values); the same loads by 64-bit addresses.
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr int DW_OFF = 7;    // offsets per wave
 constexpr int DW_ROWS = 9 * 4 * 10;   // staged x rows of a tile: (dz, dy) x octet x (x - 1 .. x + 8)
-constexpr unsigned NOWHERE = 1u << 31;
 __host__ __device__ inline long dw_window(const Shape& S, int cin, long chunk) {   // bytes of x a chunk may touch
     return (chunk + 8 + 2 * ((long)S.h * S.w + S.w + 1)) * cin * 2;
 }
@@ -529,6 +714,29 @@ extern "C" int mflbm_nn_conv3d_fwd(const void* x, const void* wf, const float* b
     if (!x || !wf || !y || n < 1 || d < 1 || h < 1 || w < 1 || cin < 8 || cin % 8 || cout < 1) return MFLBM_ERR_ARG;
     const Shape S{n, d, h, w};
     const long M = S.count();
+    hipStream_t st = (hipStream_t)stream;
+    const int kp = kpad_of(cin);
+    // Tile by channels (what fits 160 KB of LDS with the whole cin) and by the number of work-groups: the large tiles
+    // read less halo and fewer fragments per product, but need 256 work-groups to use every compute unit.  Without the
+    // tile (more than 256 input channels, or planes beyond a 2 GiB window): k_conv_fwd.
+    if (cin <= 256 && 10L * h * w * cin * 2 < (1L << 31) && (long)cout * kp * 2 < (1L << 31)) {
+        const long tiles8 = (long)n * ((d + 7) / 8) * ((h + 7) / 8) * ((w + 7) / 8);   // 8 x 8 x 8 tiles
+#define TILE(...) launch_conv_tile<__VA_ARGS__>(x, wf, bias, y, S, (int)cin, (int)cout, kp, (int)relu, st)
+        // fragments of positions and of channels, waves along positions and channels, tile, steps per weight stage
+        if (cin <= 32) {   // 4 x 64^3, us before / after: 8 -> 32 75 / 44, 32 -> 8 196 / 85, 32 -> 32 254 / 116, 32 -> 64 483 / 175
+            if (cout <= 16) return TILE(2, 1, 8, 1, 4, 8, 8, 8);
+            if (cout > 32) return TILE(4, 4, 4, 1, 4, 8, 8, 1);
+            if (cin <= 16) return TILE(4, 2, 4, 1, 4, 8, 8, 4);
+            return TILE(2, 2, 8, 1, 4, 8, 8, 4);
+        }
+        if (cin <= 64) {   // 4 x 64^3 64 -> 32 782 / 204; 4 x 32^3 64 -> 64 206 / 46 (61 in the small tile); 4 x 16^3 64 -> 128 52 / 23 (40 in the large)
+            if (cout <= 32) return tiles8 >= 256 ? TILE(4, 2, 8, 1, 8, 8, 8, 4) : TILE(2, 2, 8, 1, 4, 8, 8, 4);
+            return tiles8 * ((cout + 63) / 64) >= 256 ? TILE(4, 4, 8, 1, 8, 8, 8, 2) : TILE(2, 2, 4, 2, 4, 4, 8, 4);
+        }
+        if (cin <= 128) return TILE(2, 2, 4, 2, 4, 4, 8, 8);   // 4 x 16^3 128 -> 128 100 / 36, 4 x 32^3 128 -> 64 400 / 139
+        return TILE(1, 2, 4, 2, 4, 4, 4, 4);                   // 4 x 8^3 256 -> 256 125 / 57, 4 x 16^3 256 -> 128 195 / 118
+#undef TILE
+    }
     const dim3 grid((unsigned)((M + 127) / 128), (unsigned)((cout + 31) / 32));
     if (relu)
         hipLaunchKernelGGL(k_conv_fwd<1>, grid, dim3(NT), 0, (hipStream_t)stream, (const __bf16*)x, (const __bf16*)wf,
