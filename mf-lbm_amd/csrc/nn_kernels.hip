@@ -588,17 +588,32 @@ __global__ void __launch_bounds__(NT) k_sum_slices(const float* __restrict__ par
     out[e] += s;
 }
 
+// Elementwise kernels: V = 8 consecutive values per thread (16-byte accesses; the launchers take it where the channel
+// count or length is a multiple of 8 and every tensor starts on 16 bytes), else V = 1.  Bound by HBM; one 2-byte value per
+// thread was bound by the number of accesses instead (ReLU gradient, mean over the layers of a training step: 23 us, 13 us so; addition 29 and 15).
+template <int V>
+struct alignas(2 * V) Pack {
+    __bf16 v[V];
+};
+template <int V>
 __global__ void k_relu_bwd(__bf16* __restrict__ g, const __bf16* __restrict__ y, long n) {
     const long i = (long)blockIdx.x * NT + threadIdx.x;
-    if (i < n && !(bf2f(y[i]) > 0.f)) g[i] = f2bf(0.f);
+    if (i * V >= n) return;
+    Pack<V> a = ((const Pack<V>*)g)[i];
+    const Pack<V> b = ((const Pack<V>*)y)[i];
+#pragma unroll
+    for (int k = 0; k < V; ++k)
+        if (!(bf2f(b.v[k]) > 0.f)) a.v[k] = f2bf(0.f);
+    ((Pack<V>*)g)[i] = a;
 }
 
-// 2x average pooling (fine shape S, coarse S/2) and its adjoint; nearest 2x upsampling and its adjoint
-__global__ void k_pool2(const __bf16* __restrict__ x, __bf16* __restrict__ y, Shape S, int c, int bwd) {
-    const long i = (long)blockIdx.x * NT + threadIdx.x;
+// 2x average pooling (fine shape S, coarse S/2) and its adjoint; nearest 2x upsampling and its adjoint.  One thread per
+// V channels of a coarse position, c counted in units of V.
+template <int V>
+__device__ __forceinline__ bool coarse_at(const Shape& S, int c, long& i, long (&fine)[8]) {
+    i = (long)blockIdx.x * NT + threadIdx.x;
     const int D = S.d / 2, H = S.h / 2, W = S.w / 2;
-    const long n = (long)S.n * D * H * W * c;
-    if (i >= n) return;
+    if (i >= (long)S.n * D * H * W * c) return false;
     const int ch = (int)(i % c);
     long t = i / c;
     const int xx = (int)(t % W);
@@ -607,53 +622,72 @@ __global__ void k_pool2(const __bf16* __restrict__ x, __bf16* __restrict__ y, Sh
     t /= H;
     const int zz = (int)(t % D);
     const int nn = (int)(t / D);
-    float s = 0.f;
-    for (int o = 0; o < 8; ++o) {
-        const long f = ((((long)nn * S.d + 2 * zz + (o >> 2)) * S.h + 2 * yy + ((o >> 1) & 1)) * S.w + 2 * xx + (o & 1)) * c + ch;
-        if (!bwd) s += bf2f(x[f]);
-        else y[f] = f2bf(0.125f * bf2f(x[i]));   // x: coarse gradient, y: fine gradient
-    }
-    if (!bwd) y[i] = f2bf(0.125f * s);
+#pragma unroll
+    for (int o = 0; o < 8; ++o)
+        fine[o] = ((((long)nn * S.d + 2 * zz + (o >> 2)) * S.h + 2 * yy + ((o >> 1) & 1)) * S.w + 2 * xx + (o & 1)) * c + ch;
+    return true;
 }
-__global__ void k_up2(const __bf16* __restrict__ x, __bf16* __restrict__ y, Shape S, int c, int bwd) {
-    // S: fine shape.  forward: y(fine) = x(coarse parent); backward: y(coarse) = sum of x(fine children)
-    const long i = (long)blockIdx.x * NT + threadIdx.x;
-    const int D = S.d / 2, H = S.h / 2, W = S.w / 2;
-    const long n = (long)S.n * D * H * W * c;
-    if (i >= n) return;
-    const int ch = (int)(i % c);
-    long t = i / c;
-    const int xx = (int)(t % W);
-    t /= W;
-    const int yy = (int)(t % H);
-    t /= H;
-    const int zz = (int)(t % D);
-    const int nn = (int)(t / D);
-    float s = 0.f;
-    for (int o = 0; o < 8; ++o) {
-        const long f = ((((long)nn * S.d + 2 * zz + (o >> 2)) * S.h + 2 * yy + ((o >> 1) & 1)) * S.w + 2 * xx + (o & 1)) * c + ch;
-        if (bwd) s += bf2f(x[f]);
-        else y[f] = x[i];
+// SUM: the sum of the fine values (scaled by 1/8 as pooling, unscaled as the upsampling's adjoint); else each fine value
+// takes the coarse one (scaled by 1/8 as the pooling's adjoint)
+template <int V, bool SUM, bool EIGHTH>
+__global__ void k_coarse(const __bf16* __restrict__ x, __bf16* __restrict__ y, Shape S, int c) {
+    long i, f[8];
+    if (!coarse_at<V>(S, c, i, f)) return;
+    const Pack<V>* const X = (const Pack<V>*)x;
+    Pack<V>* const Y = (Pack<V>*)y;
+    if (SUM) {
+        Pack<V> a[8], r;
+#pragma unroll
+        for (int o = 0; o < 8; ++o) a[o] = X[f[o]];
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            float s = 0.f;
+#pragma unroll
+            for (int o = 0; o < 8; ++o) s += bf2f(a[o].v[k]);
+            r.v[k] = f2bf(EIGHTH ? 0.125f * s : s);
+        }
+        Y[i] = r;
+    } else {
+        Pack<V> a = X[i];
+        if (EIGHTH) {
+#pragma unroll
+            for (int k = 0; k < V; ++k) a.v[k] = f2bf(0.125f * bf2f(a.v[k]));
+        }
+#pragma unroll
+        for (int o = 0; o < 8; ++o) Y[f[o]] = a;
     }
-    if (bwd) y[i] = f2bf(s);
 }
+template <int V>
 __global__ void k_add(const __bf16* __restrict__ a, const __bf16* __restrict__ b, __bf16* __restrict__ y, long n) {
     const long i = (long)blockIdx.x * NT + threadIdx.x;
-    if (i < n) y[i] = f2bf(bf2f(a[i]) + bf2f(b[i]));
+    if (i * V >= n) return;
+    const Pack<V> u = ((const Pack<V>*)a)[i], w = ((const Pack<V>*)b)[i];
+    Pack<V> r;
+#pragma unroll
+    for (int k = 0; k < V; ++k) r.v[k] = f2bf(bf2f(u.v[k]) + bf2f(w.v[k]));
+    ((Pack<V>*)y)[i] = r;
 }
 // mean squared error over the first `used` of `c` channels; writes the gradient (BF16) and adds the sum of
-// squares to *loss (FP32)
+// squares to *loss (FP32).  At most MSE_BLOCKS work-groups walk the tensor: one atomic addition to the one address per
+// 256 values took 420 us of a training step (4 x 64^3 x 8), under 15 us so.
+constexpr int MSE_BLOCKS = 1024;
+template <int V>
 __global__ void __launch_bounds__(NT) k_mse(const __bf16* __restrict__ y, const __bf16* __restrict__ t,
-                                            __bf16* __restrict__ g, float* __restrict__ loss, long npos, int c, int used,
+                                            __bf16* __restrict__ g, float* __restrict__ loss, long n, int c, int used,
                                             float scale) {
-    const long i = (long)blockIdx.x * NT + threadIdx.x;
     __shared__ float red[NT];
     float s = 0.f;
-    if (i < npos * c) {
-        const int ch = (int)(i % c);
-        const float d = ch < used ? bf2f(y[i]) - bf2f(t[i]) : 0.f;
-        g[i] = f2bf(2.f * scale * d);
-        s = d * d;
+    for (long i = (long)blockIdx.x * NT + threadIdx.x; i * V < n; i += (long)gridDim.x * NT) {
+        const Pack<V> a = ((const Pack<V>*)y)[i], b = ((const Pack<V>*)t)[i];
+        Pack<V> r;
+        const int ch = (int)(i * V % c);
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            const float d = ch + k < used ? bf2f(a.v[k]) - bf2f(b.v[k]) : 0.f;
+            r.v[k] = f2bf(2.f * scale * d);
+            s += d * d;
+        }
+        ((Pack<V>*)g)[i] = r;
     }
     red[threadIdx.x] = s;
     __syncthreads();
@@ -853,9 +887,19 @@ extern "C" int mflbm_nn_weights_to_bf16(const float* w, void* wf, void* wb, int3
     return launched((hipStream_t)stream);
 }
 
+namespace {
+// every tensor on a 16-byte boundary and the length (or channel count) whole packs of 8
+template <class... P>
+bool packs(long n, const P*... p) {
+    return n % 8 == 0 && (... && (((uintptr_t)p & 15) == 0));
+}
+}  // namespace
+
 extern "C" int mflbm_nn_relu_bwd(void* g, const void* y, int64_t n, void* stream) {
     if (!g || !y || n < 0) return MFLBM_ERR_ARG;
-    if (n) hipLaunchKernelGGL(k_relu_bwd, dim3(blocks(n)), dim3(NT), 0, (hipStream_t)stream, (__bf16*)g, (const __bf16*)y, (long)n);
+    const bool v = packs(n, (const char*)g, (const char*)y);
+    if (n) hipLaunchKernelGGL(v ? k_relu_bwd<8> : k_relu_bwd<1>, dim3(blocks(v ? n / 8 : n)), dim3(NT), 0, (hipStream_t)stream,
+                              (__bf16*)g, (const __bf16*)y, (long)n);
     return launched((hipStream_t)stream);
 }
 
@@ -922,30 +966,37 @@ extern "C" int mflbm_nn_distance_features(const int8_t* fluid, int32_t* work, vo
     return launched(st);
 }
 
+namespace {
+template <bool SUM, bool EIGHTH>
+int launch_coarse(const void* x, void* y, const Shape& S, int c, hipStream_t st) {
+    const bool v = packs(c, (const char*)x, (const char*)y);
+    const int cv = v ? c / 8 : c;
+    const long cnt = (long)S.n * (S.d / 2) * (S.h / 2) * (S.w / 2) * cv;
+    hipLaunchKernelGGL((v ? k_coarse<8, SUM, EIGHTH> : k_coarse<1, SUM, EIGHTH>), dim3(blocks(cnt)), dim3(NT), 0, st,
+                       (const __bf16*)x, (__bf16*)y, S, cv);
+    return launched(st);
+}
+}  // namespace
+
 extern "C" int mflbm_nn_pool2(const void* x, void* y, int32_t n, int32_t d, int32_t h, int32_t w, int32_t c, int32_t bwd,
                               void* stream) {
     if (!x || !y || d % 2 || h % 2 || w % 2 || c < 1) return MFLBM_ERR_ARG;
     const Shape S{n, d, h, w};
-    const long cnt = (long)n * (d / 2) * (h / 2) * (w / 2) * c;
-    hipLaunchKernelGGL(k_pool2, dim3(blocks(cnt)), dim3(NT), 0, (hipStream_t)stream, (const __bf16*)x, (__bf16*)y, S, (int)c,
-                       (int)bwd);
-    return launched((hipStream_t)stream);
+    return bwd ? launch_coarse<false, true>(x, y, S, c, (hipStream_t)stream) : launch_coarse<true, true>(x, y, S, c, (hipStream_t)stream);
 }
 
 extern "C" int mflbm_nn_up2(const void* x, void* y, int32_t n, int32_t d, int32_t h, int32_t w, int32_t c, int32_t bwd,
                             void* stream) {
     if (!x || !y || d % 2 || h % 2 || w % 2 || c < 1) return MFLBM_ERR_ARG;
     const Shape S{n, d, h, w};
-    const long cnt = (long)n * (d / 2) * (h / 2) * (w / 2) * c;
-    hipLaunchKernelGGL(k_up2, dim3(blocks(cnt)), dim3(NT), 0, (hipStream_t)stream, (const __bf16*)x, (__bf16*)y, S, (int)c,
-                       (int)bwd);
-    return launched((hipStream_t)stream);
+    return bwd ? launch_coarse<true, false>(x, y, S, c, (hipStream_t)stream) : launch_coarse<false, false>(x, y, S, c, (hipStream_t)stream);
 }
 
 extern "C" int mflbm_nn_add(const void* a, const void* b, void* y, int64_t n, void* stream) {
     if (!a || !b || !y || n < 0) return MFLBM_ERR_ARG;
-    if (n) hipLaunchKernelGGL(k_add, dim3(blocks(n)), dim3(NT), 0, (hipStream_t)stream, (const __bf16*)a, (const __bf16*)b,
-                              (__bf16*)y, (long)n);
+    const bool v = packs(n, (const char*)a, (const char*)b, (const char*)y);
+    if (n) hipLaunchKernelGGL(v ? k_add<8> : k_add<1>, dim3(blocks(v ? n / 8 : n)), dim3(NT), 0, (hipStream_t)stream,
+                              (const __bf16*)a, (const __bf16*)b, (__bf16*)y, (long)n);
     return launched((hipStream_t)stream);
 }
 
@@ -953,8 +1004,10 @@ extern "C" int mflbm_nn_mse(const void* y, const void* t, void* g, float* loss, 
                             float scale, void* stream) {
     if (!y || !t || !g || !loss || npos < 0 || c < 1 || used < 0 || used > c) return MFLBM_ERR_ARG;
     const long n = (long)npos * c;
-    if (n) hipLaunchKernelGGL(k_mse, dim3(blocks(n)), dim3(NT), 0, (hipStream_t)stream, (const __bf16*)y, (const __bf16*)t,
-                              (__bf16*)g, loss, (long)npos, (int)c, (int)used, scale);
+    const bool v = packs(c, (const char*)y, (const char*)t, (const char*)g);
+    const unsigned nb = blocks(v ? n / 8 : n);
+    if (n) hipLaunchKernelGGL(v ? k_mse<8> : k_mse<1>, dim3(nb < MSE_BLOCKS ? nb : MSE_BLOCKS), dim3(NT), 0, (hipStream_t)stream,
+                              (const __bf16*)y, (const __bf16*)t, (__bf16*)g, loss, n, (int)c, (int)used, scale);
     return launched((hipStream_t)stream);
 }
 
