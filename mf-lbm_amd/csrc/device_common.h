@@ -88,17 +88,29 @@ __device__ __forceinline__ void odd_neighbour_slots(const RowRec* rows_, const L
     }
 }
 
+// Whether the even step of a state of these bytes (fluid nodes only) reads and writes its slots non-temporally.  The
+// even step touches every slot line once, whole: beyond what the 256 MB last-level cache keeps from step to step its
+// lines only push out those that are read again (the odd step's shared lines, normals, phi, row records).  us per step
+// (even and odd mean), cached / streamed: two-phase FP64 90 MB 71 / 77, 196 MB 137 / 130, 362 MB 247 / 211, 1349 MB
+// 791 / 723; FP32 181 MB 185 / 172; single-phase FP64 98 MB 37 / 39, 181 MB 77 / 69, 674 MB 307 / 273; FP32 150 MB
+// 54 / 61, 231 MB 110 / 95, 337 MB 159 / 140.  (The odd step's lines are shared by neighbouring rows: streamed loads
+// took its 256^3 update from 689 to 923 us, streamed stores to 698.)
+inline bool stream_even(long pop_bytes) { return pop_bytes > (160L << 20); }
+
 // Slot access with a scalar slice base and a 32-bit per-lane byte offset (one global load/store with an SGPR
 // base instead of a 64-bit vector address per slot); slices are kept below 2^32 bytes.
-template <class T>
+// STREAM: a non-temporal access, for the even step of a state that no cache holds (stream_even).
+template <bool STREAM = false, class T>
 __device__ __forceinline__ T slot_ld(const T* slice, unsigned i) {
-    return *(const MFLBM_GLOBAL T*)((const MFLBM_GLOBAL char*)slice + i * (unsigned)sizeof(T));
+    const MFLBM_GLOBAL T* const p = (const MFLBM_GLOBAL T*)((const MFLBM_GLOBAL char*)slice + i * (unsigned)sizeof(T));
+    return STREAM ? __builtin_nontemporal_load(p) : *p;
 }
-template <class T>
+template <bool STREAM = false, class T>
 __device__ __forceinline__ void slot_st(T* slice, unsigned i, T v) {
-    *(MFLBM_GLOBAL T*)((MFLBM_GLOBAL char*)slice + i * (unsigned)sizeof(T)) = v;
+    MFLBM_GLOBAL T* const p = (MFLBM_GLOBAL T*)((MFLBM_GLOBAL char*)slice + i * (unsigned)sizeof(T));
+    if (STREAM) __builtin_nontemporal_store(v, p);
+    else *p = v;
 }
-
 // Exchanged halo slots of a folded domain (layout.h, Fold): the halo slot (q, h) of a direction q that points
 // into the domain along h's halo axes, and the slot (q, y) of h's image.  The reference's self-exchange leaves them
 // equal after every step.

@@ -214,17 +214,19 @@ struct PhiNowAt {
 // upload_geometry guarantees that every slice is below 2^32 bytes.
 // The two colours of a slot are adjacent (f_q, g_q or s_q, a_q): one 16-byte (FP64) or 8-byte (FP32) access
 // moves both, which halves the scattered accesses of the odd step.
-__device__ __forceinline__ double2 ld_pair(const double* slice, unsigned m) {
-    return *(const double2*)((const char*)slice + m * 16u);
-}
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+template <bool STREAM = false>
+__device__ __forceinline__ d2 ld_pair(const double* slice, unsigned m) { return slot_ld<STREAM>((const d2*)slice, m); }
+template <bool STREAM = false>
 __device__ __forceinline__ void st_pair(double* slice, unsigned m, double f, double g) {
-    *(double2*)((char*)slice + m * 16u) = double2{f, g};
+    slot_st<STREAM>((d2*)slice, m, d2{f, g});
 }
-__device__ __forceinline__ float2 ld_pair32(const double* slice, unsigned m) {
-    return *(const float2*)((const char*)slice + m * 8u);
-}
+template <bool STREAM = false>
+__device__ __forceinline__ f2 ld_pair32(const double* slice, unsigned m) { return slot_ld<STREAM>((const f2*)slice, m); }
+template <bool STREAM = false>
 __device__ __forceinline__ void st_pair32(double* slice, unsigned m, float s, float a) {
-    *(float2*)((char*)slice + m * 8u) = float2{s, a};
+    slot_st<STREAM>((f2*)slice, m, f2{s, a});
 }
 // One slot (direction q, index i) of both colours held in registers.  The velocity inlet and the convective outlet
 // load every slot they touch before their first store (a load after a store through another pointer of the same
@@ -299,7 +301,7 @@ __device__ __forceinline__ double quiet_curvature();
 // The CSF force input (curvature, Phase_gradient.F90:112-201, and 0.5*gamma*curv*c_norm,
 // Kernel_multiphase.F90:116) is either evaluated here from the dense normal field the list kernels of the chain
 // left (STENCIL), or read from the compact force arrays the fused chain (k_chain_force) wrote.
-template <bool ODD, bool STENCIL>
+template <bool ODD, bool STENCIL, bool STREAM>
 __global__ void __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(2, 8)))
 k_collide(Dev d, CollideParams P, int per) {
@@ -332,7 +334,7 @@ k_collide(Dev d, CollideParams P, int per) {
     double a[19], b[19];
     unsigned nb[19];   // odd: per direction r, the index of the slot (x + e_r, opp(r)) in slice opp(r)
     {
-        const double2 v = ld_pair(S.p[0], m);
+        const d2 v = ld_pair<STREAM>(S.p[0], m);
         a[0] = v.x;
         b[0] = v.y;
     }
@@ -340,14 +342,14 @@ k_collide(Dev d, CollideParams P, int per) {
         odd_neighbour_slots(d.rows, d.L, d.nc, d.wbase, d.wmask, m, nn, nb);
 #pragma unroll
         for (int q = 1; q < 19; ++q) {   // slot q of the upwind node x - e_q = x + e_opp(q)
-            const double2 v = ld_pair(S.p[q], nb[lat::OPP[q]]);
+            const d2 v = ld_pair(S.p[q], nb[lat::OPP[q]]);
             a[q] = v.x;
             b[q] = v.y;
         }
     } else {
 #pragma unroll
         for (int q = 1; q < 19; ++q) {
-            const double2 v = ld_pair(S.p[lat::OPP[q]], m);
+            const d2 v = ld_pair<STREAM>(S.p[lat::OPP[q]], m);
             a[q] = v.x;
             b[q] = v.y;
         }
@@ -355,19 +357,19 @@ k_collide(Dev d, CollideParams P, int per) {
     const double phi = collide_node_tf(a, b, cnx, cny, cnz, tf, P);
     flag_band(d, brick_of(d, nn), phi);
     d.phic[m] = phi;
-    st_pair(S.p[0], m, a[0], b[0]);
+    st_pair<STREAM>(S.p[0], m, a[0], b[0]);
 #pragma unroll
     for (int q = 1; q < 19; ++q) {   // odd: slot opp(q) of x + e_q
         const int qs = ODD ? lat::OPP[q] : q;
         const unsigned ms = ODD ? nb[q] : (unsigned)m;
-        st_pair(S.p[qs], ms, a[q], b[q]);
+        st_pair<STREAM>(S.p[qs], ms, a[q], b[q]);
     }
 }
 
 // FP32 storage (s = f + g - REST, a = f - g, collide.h): the same update, the collision and recolouring in C
 // (float, or double for the mixed mode).  The normal, curvature and phi stay FP64 (the colour-gradient chain is
 // shared with the FP64 path).
-template <bool ODD, class C, bool STENCIL>
+template <bool ODD, class C, bool STENCIL, bool STREAM>
 __global__ void __launch_bounds__(BLOCK) k_collide32(Dev d, CollideParamsDev<C> P, double gamma, int per) {
     const SlotTable& S = d.S;
     const int m = (int)blockIdx.x * BLOCK + (int)threadIdx.x;
@@ -397,7 +399,7 @@ __global__ void __launch_bounds__(BLOCK) k_collide32(Dev d, CollideParamsDev<C> 
     C s[19], a[19];
     unsigned nb[19];
     {
-        const float2 v = ld_pair32(S.p[0], (unsigned)m);
+        const f2 v = ld_pair32<STREAM>(S.p[0], (unsigned)m);
         s[0] = v.x;
         a[0] = v.y;
     }
@@ -405,14 +407,14 @@ __global__ void __launch_bounds__(BLOCK) k_collide32(Dev d, CollideParamsDev<C> 
         odd_neighbour_slots(d.rows, d.L, d.nc, d.wbase, d.wmask, m, nn, nb);
 #pragma unroll
         for (int q = 1; q < 19; ++q) {
-            const float2 v = ld_pair32(S.p[q], nb[lat::OPP[q]]);
+            const f2 v = ld_pair32(S.p[q], nb[lat::OPP[q]]);
             s[q] = v.x;
             a[q] = v.y;
         }
     } else {
 #pragma unroll
         for (int q = 1; q < 19; ++q) {
-            const float2 v = ld_pair32(S.p[lat::OPP[q]], (unsigned)m);
+            const f2 v = ld_pair32<STREAM>(S.p[lat::OPP[q]], (unsigned)m);
             s[q] = v.x;
             a[q] = v.y;
         }
@@ -420,12 +422,12 @@ __global__ void __launch_bounds__(BLOCK) k_collide32(Dev d, CollideParamsDev<C> 
     const C phi = collide_node_dev<C>(s, a, cnx, cny, cnz, tf, P);
     flag_band(d, brick_of(d, nn), (double)phi);
     d.phic[m] = (double)phi;
-    st_pair32(S.p[0], (unsigned)m, (float)s[0], (float)a[0]);
+    st_pair32<STREAM>(S.p[0], (unsigned)m, (float)s[0], (float)a[0]);
 #pragma unroll
     for (int q = 1; q < 19; ++q) {
         const int qs = ODD ? lat::OPP[q] : q;
         const unsigned ms = ODD ? nb[q] : (unsigned)m;
-        st_pair32(S.p[qs], ms, (float)s[q], (float)a[q]);
+        st_pair32<STREAM>(S.p[qs], ms, (float)s[q], (float)a[q]);
     }
 }
 
@@ -2211,28 +2213,28 @@ int launch_step(mflbm_ctx* c, int ntime) {
         HIPCHK(c, hipEventRecord(ev[0], c->stream));
     }
     const int per = xcd_per(c->d.nf);
-#define MFLBM_COLLIDE32(C_, PP)                                                                                  \
-    if (c->chain_fused) {                                                                                        \
-        if (odd) LAUNCH(c, (k_collide32<true, C_, false>), NXCD * per, c->d, PP, p.gamma, per);                   \
-        else LAUNCH(c, (k_collide32<false, C_, false>), NXCD * per, c->d, PP, p.gamma, per);                      \
-    } else {                                                                                                     \
-        if (odd) LAUNCH(c, (k_collide32<true, C_, true>), NXCD * per, c->d, PP, p.gamma, per);                    \
-        else LAUNCH(c, (k_collide32<false, C_, true>), NXCD * per, c->d, PP, p.gamma, per);                       \
-    }
+    const bool stream = !odd && stream_even(19L * c->d.nf * (c->fp32 ? 8 : 16));
+#define MFLBM_COLLIDE32(C_, PP, STENCIL)                                                                         \
+    if (odd) LAUNCH(c, (k_collide32<true, C_, STENCIL, false>), NXCD * per, c->d, PP, p.gamma, per);             \
+    else if (stream) LAUNCH(c, (k_collide32<false, C_, STENCIL, true>), NXCD * per, c->d, PP, p.gamma, per);     \
+    else LAUNCH(c, (k_collide32<false, C_, STENCIL, false>), NXCD * per, c->d, PP, p.gamma, per);
+#define MFLBM_COLLIDE(STENCIL)                                                                                   \
+    if (odd) LAUNCH(c, (k_collide<true, STENCIL, false>), NXCD * per, c->d, P, per);                             \
+    else if (stream) LAUNCH(c, (k_collide<false, STENCIL, true>), NXCD * per, c->d, P, per);                     \
+    else LAUNCH(c, (k_collide<false, STENCIL, false>), NXCD * per, c->d, P, per);
     if (c->fp32 && c->p.precision == 2) {
         const CollideParamsDev<double> PD{p.gamma, p.beta, p.force_z, p.la_nui1, p.la_nui2};
-        MFLBM_COLLIDE32(double, PD)
+        if (c->chain_fused) { MFLBM_COLLIDE32(double, PD, false) } else { MFLBM_COLLIDE32(double, PD, true) }
     } else if (c->fp32) {
         const CollideParamsDev<float> P32{(float)p.gamma, (float)p.beta, (float)p.force_z, (float)p.la_nui1, (float)p.la_nui2};
-        MFLBM_COLLIDE32(float, P32)
+        if (c->chain_fused) { MFLBM_COLLIDE32(float, P32, false) } else { MFLBM_COLLIDE32(float, P32, true) }
     } else if (c->chain_fused) {
-        if (odd) LAUNCH(c, (k_collide<true, false>), NXCD * per, c->d, P, per);
-        else LAUNCH(c, (k_collide<false, false>), NXCD * per, c->d, P, per);
+        MFLBM_COLLIDE(false)
     } else {
-        if (odd) LAUNCH(c, (k_collide<true, true>), NXCD * per, c->d, P, per);
-        else LAUNCH(c, (k_collide<false, true>), NXCD * per, c->d, P, per);
+        MFLBM_COLLIDE(true)
     }
 #undef MFLBM_COLLIDE32
+#undef MFLBM_COLLIDE
     if (t) HIPCHK(c, hipEventRecord(ev[1], c->stream));
     FaceWork faces;
     FaceWork* defer = c->chain_all ? nullptr : &faces;   // (no plan launch to take the faces)

@@ -33,7 +33,7 @@ namespace {
 constexpr int WAVE = 64;
 
 // lattice update of every active sample; global wave w covers nodes [64 (w - wave_first[s]), +64) of sample s
-template <bool ODD, class T, class C, int NT>
+template <bool ODD, bool STREAM, class T, class C, int NT>
 __global__ void __launch_bounds__(NT) k_spb_collide(const SDev<T>* __restrict__ devs, const int* __restrict__ wave_sample,
                                                     const int* __restrict__ wave_first, const int* __restrict__ active,
                                                     SPCollideParamsT<C> P, int nwaves, int per) {
@@ -44,7 +44,7 @@ __global__ void __launch_bounds__(NT) k_spb_collide(const SDev<T>* __restrict__ 
     const SDev<T> d = devs[s];   // a copy: the slice bases stay scalar across the stores
     const int m = (w - wave_first[s]) * WAVE + (int)(threadIdx.x % WAVE);
     if (m >= d.nf) return;
-    sp_update_node<ODD, T, C>(d, P, m);
+    sp_update_node<ODD, STREAM, T, C>(d, P, m);
 }
 
 // periodic self-exchange of every active sample periodic along y as well as z (the samples periodic along z only
@@ -177,6 +177,7 @@ struct mflbm_spb_ctx {
     std::vector<SDev<float>> dev32;
     int nwaves = 0;
     long nfluid = 0;
+    long pop_bytes = 0;                  // populations of the fluid nodes of all samples
     hipStream_t stream = nullptr;
     void* pop = nullptr;                 // all samples' population slices
     std::vector<void*> bufs;             // maps, cpos, link masks and bases of every sample
@@ -226,12 +227,10 @@ int launch_collide_t(mflbm_spb_ctx* c, bool odd) {
     const int per = (int)((nb + NXCD - 1) / NXCD);
     const unsigned grid = (unsigned)(NXCD * per);
     if (grid == 0) return MFLBM_OK;
-    if (odd)
-        hipLaunchKernelGGL((k_spb_collide<true, T, C, NT>), dim3(grid), dim3(NT), 0, c->stream, devs_of<T>(c),
-                           c->wave_sample, c->wave_first, c->M.active, rates_of<C>(c), c->nwaves, per);
-    else
-        hipLaunchKernelGGL((k_spb_collide<false, T, C, NT>), dim3(grid), dim3(NT), 0, c->stream, devs_of<T>(c),
-                           c->wave_sample, c->wave_first, c->M.active, rates_of<C>(c), c->nwaves, per);
+    const auto kern = odd ? k_spb_collide<true, false, T, C, NT>
+                          : stream_even(c->pop_bytes) ? k_spb_collide<false, true, T, C, NT> : k_spb_collide<false, false, T, C, NT>;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), 0, c->stream, devs_of<T>(c), c->wave_sample, c->wave_first, c->M.active,
+                       rates_of<C>(c), c->nwaves, per);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(c, MFLBM_ERR_HIP, "launch k_spb_collide: %s", hipGetErrorString(e));
     return MFLBM_OK;
@@ -446,6 +445,7 @@ extern "C" int mflbm_spb_commit(mflbm_spb_ctx* c) {
     c->nfluid = P.nfluid;
     c->nwaves = P.nwaves;
     const long elems = P.elems, maxdense = P.maxdense;
+    c->pop_bytes = 19L * esz * P.nfluid;
     const int waves = P.nwaves;
     // device buffers
     HIPCHK(c, hipMalloc(&c->pop, (size_t)(esz * std::max(elems, 1L))));

@@ -88,18 +88,18 @@ __device__ __forceinline__ int plane_at(const SDev<T>& d, int i, int j) { return
 // The update of fluid node m (compact index, m < nf).  m & 63 must be the node's lane in its wave and all
 // lanes of a wave must belong to the same sample: the link masks are per wave of 64 consecutive nodes.
 // T is the storage type, C the arithmetic of the collision (C = T, or FP32 storage with an FP64 collision).
-template <bool ODD, class T, class C>
+template <bool ODD, bool STREAM, class T, class C>
 __device__ __forceinline__ void sp_update_node(const SDev<T>& d, const SPCollideParamsT<C>& P, int m) {
     T a[19];
     unsigned nb[19];   // odd: per direction r, the index of the slot (x + e_r, opp(r)) in slice opp(r)
-    a[0] = slot_ld(d.S[0], m);
+    a[0] = slot_ld<STREAM>(d.S[0], m);
     if (ODD) {
         odd_neighbour_slots(d.rows, d.L, d.nc, d.wbase, d.wmask, m, slot_ld(d.cpos, (unsigned)m), nb);
 #pragma unroll
         for (int q = 1; q < 19; ++q) a[q] = slot_ld(d.S[q], nb[lat::OPP[q]]);   // slot q of the upwind node x - e_q
     } else {
 #pragma unroll
-        for (int q = 1; q < 19; ++q) a[q] = slot_ld(d.S[lat::OPP[q]], m);
+        for (int q = 1; q < 19; ++q) a[q] = slot_ld<STREAM>(d.S[lat::OPP[q]], m);
     }
     if (sizeof(C) == sizeof(T)) {
         collide_single<C>((C*)a, P);
@@ -111,20 +111,20 @@ __device__ __forceinline__ void sp_update_node(const SDev<T>& d, const SPCollide
 #pragma unroll
         for (int q = 0; q < 19; ++q) a[q] = (T)w[q];
     }
-    slot_st(d.S[0], m, a[0]);
+    slot_st<STREAM>(d.S[0], m, a[0]);
 #pragma unroll
     for (int q = 1; q < 19; ++q) {
         if (ODD) slot_st(d.S[lat::OPP[q]], nb[q], a[q]);   // slot opp(q) of x + e_q
-        else slot_st(d.S[q], m, a[q]);
+        else slot_st<STREAM>(d.S[q], m, a[q]);
     }
 }
 
 // block order: plain for FP64 storage, XCD-aware for FP32 storage (each measured the faster at 256^3, by 2 %)
-template <bool ODD, class T, class C>
+template <bool ODD, bool STREAM, class T, class C>
 __global__ void __launch_bounds__(BLOCK) k_sp_collide(SDev<T> d, SPCollideParamsT<C> P, int per) {
     const int m = (sizeof(T) == sizeof(double) ? (int)blockIdx.x : xcd_block(per)) * BLOCK + (int)threadIdx.x;
     if (m >= d.nf) return;
-    sp_update_node<ODD, T, C>(d, P, m);
+    sp_update_node<ODD, STREAM, T, C>(d, P, m);
 }
 
 // dense staging (populations f, FP64) <-> compact storage
