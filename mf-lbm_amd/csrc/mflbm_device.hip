@@ -304,9 +304,9 @@ __device__ __forceinline__ double quiet_curvature();
 template <bool ODD, bool STENCIL, bool STREAM>
 __global__ void __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(2, 8)))
-k_collide(Dev d, CollideParams P, int per) {
+k_collide(Dev d, CollideParams P) {
     const SlotTable& S = d.S;
-    const int m = (int)blockIdx.x * BLOCK + (int)threadIdx.x;
+    const int m = (ODD ? odd_block() : (int)blockIdx.x) * BLOCK + (int)threadIdx.x;
     if (m >= d.nf) return;
     const int nn = d.cpos[m];
     double cnx, cny, cnz, tf;
@@ -370,9 +370,9 @@ k_collide(Dev d, CollideParams P, int per) {
 // (float, or double for the mixed mode).  The normal, curvature and phi stay FP64 (the colour-gradient chain is
 // shared with the FP64 path).
 template <bool ODD, class C, bool STENCIL, bool STREAM>
-__global__ void __launch_bounds__(BLOCK) k_collide32(Dev d, CollideParamsDev<C> P, double gamma, int per) {
+__global__ void __launch_bounds__(BLOCK) k_collide32(Dev d, CollideParamsDev<C> P, double gamma) {
     const SlotTable& S = d.S;
-    const int m = (int)blockIdx.x * BLOCK + (int)threadIdx.x;
+    const int m = (ODD ? odd_block() : (int)blockIdx.x) * BLOCK + (int)threadIdx.x;
     if (m >= d.nf) return;
     const int nn = d.cpos[m];
     C cnx, cny, cnz, tf;
@@ -2212,16 +2212,16 @@ int launch_step(mflbm_ctx* c, int ntime) {
         c->ev_used += 4;
         HIPCHK(c, hipEventRecord(ev[0], c->stream));
     }
-    const int per = xcd_per(c->d.nf);
+    const unsigned nb = nblocks(c->d.nf), nbo = odd_grid(nb);
     const bool stream = !odd && stream_even(19L * c->d.nf * (c->fp32 ? 8 : 16));
 #define MFLBM_COLLIDE32(C_, PP, STENCIL)                                                                         \
-    if (odd) LAUNCH(c, (k_collide32<true, C_, STENCIL, false>), NXCD * per, c->d, PP, p.gamma, per);             \
-    else if (stream) LAUNCH(c, (k_collide32<false, C_, STENCIL, true>), NXCD * per, c->d, PP, p.gamma, per);     \
-    else LAUNCH(c, (k_collide32<false, C_, STENCIL, false>), NXCD * per, c->d, PP, p.gamma, per);
+    if (odd) LAUNCH(c, (k_collide32<true, C_, STENCIL, false>), nbo, c->d, PP, p.gamma);             \
+    else if (stream) LAUNCH(c, (k_collide32<false, C_, STENCIL, true>), nb, c->d, PP, p.gamma);     \
+    else LAUNCH(c, (k_collide32<false, C_, STENCIL, false>), nb, c->d, PP, p.gamma);
 #define MFLBM_COLLIDE(STENCIL)                                                                                   \
-    if (odd) LAUNCH(c, (k_collide<true, STENCIL, false>), NXCD * per, c->d, P, per);                             \
-    else if (stream) LAUNCH(c, (k_collide<false, STENCIL, true>), NXCD * per, c->d, P, per);                     \
-    else LAUNCH(c, (k_collide<false, STENCIL, false>), NXCD * per, c->d, P, per);
+    if (odd) LAUNCH(c, (k_collide<true, STENCIL, false>), nbo, c->d, P);                             \
+    else if (stream) LAUNCH(c, (k_collide<false, STENCIL, true>), nb, c->d, P);                     \
+    else LAUNCH(c, (k_collide<false, STENCIL, false>), nb, c->d, P);
     if (c->fp32 && c->p.precision == 2) {
         const CollideParamsDev<double> PD{p.gamma, p.beta, p.force_z, p.la_nui1, p.la_nui2};
         if (c->chain_fused) { MFLBM_COLLIDE32(double, PD, false) } else { MFLBM_COLLIDE32(double, PD, true) }

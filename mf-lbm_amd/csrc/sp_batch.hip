@@ -37,7 +37,7 @@ template <bool ODD, bool STREAM, class T, class C, int NT>
 __global__ void __launch_bounds__(NT) k_spb_collide(const SDev<T>* __restrict__ devs, const int* __restrict__ wave_sample,
                                                     const int* __restrict__ wave_first, const int* __restrict__ active,
                                                     SPCollideParamsT<C> P, int nwaves, int per) {
-    const int w = xcd_block(per) * (NT / WAVE) + (int)(threadIdx.x / WAVE);
+    const int w = (ODD ? odd_block() : xcd_block(per)) * (NT / WAVE) + (int)(threadIdx.x / WAVE);
     if (w >= nwaves) return;
     const int s = __builtin_amdgcn_readfirstlane(wave_sample[w]);
     if (!active[s]) return;
@@ -225,7 +225,7 @@ template <class T, class C, int NT>
 int launch_collide_t(mflbm_spb_ctx* c, bool odd) {
     const long nb = ((long)c->nwaves * WAVE + NT - 1) / NT;
     const int per = (int)((nb + NXCD - 1) / NXCD);
-    const unsigned grid = (unsigned)(NXCD * per);
+    const unsigned grid = odd ? odd_grid(nb) : (unsigned)(NXCD * per);
     if (grid == 0) return MFLBM_OK;
     const auto kern = odd ? k_spb_collide<true, false, T, C, NT>
                           : stream_even(c->pop_bytes) ? k_spb_collide<false, true, T, C, NT> : k_spb_collide<false, false, T, C, NT>;
