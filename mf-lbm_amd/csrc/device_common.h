@@ -36,21 +36,24 @@ constexpr int NXCD = 8;   // gfx950: 8 accelerator complex dies, work-groups dis
 
 // Logical block index with each XCD taking one contiguous range of blocks: node lists are in x-fastest
 // order, so a die then works on a z-slab and stencil neighbours stay in its own L2.  The grid is launched
-// as NXCD * per blocks.  (The FP64 and two-phase even steps use the plain block order instead: with every die streaming
-// its own distant range, they ran 2 % slower at 256^3, the populations having no reuse to gain from the L2.)
+// as NXCD * per blocks.  (The lattice updates take update_block.)
 __device__ __forceinline__ int xcd_block(int per) { return (int)(blockIdx.x % NXCD) * per + (int)(blockIdx.x / NXCD); }
 
-// Logical block index of the odd step: the dies take runs of ODD_RUN consecutive blocks in turn.  A slot line is shared
-// by the rows its run boundaries fall on (neighbouring blocks) and read by the planes above and below (some 8 blocks on),
-// so a run keeps most sharers on one die's L2, while all dies still stream one region.  Odd step, us, runs of 1 / 8 / 32
-// / 128 blocks: two-phase 256^3 FP64 665 / 653 / 652 / 685, 160^3 FP32 89 / 85 / 84 / 88, single-phase 160^3 FP64 88 / 81
-// / 81 / 84 (whole eighths: 88), 125x131x119 FP32 21.7 / 20.0 / 20.0 / 20.1.  The grid is odd_grid(blocks).
-constexpr int ODD_RUN = 16;
-__device__ __forceinline__ int odd_block() {
+// Logical block index of the lattice updates: the dies take runs of UPDATE_RUN consecutive blocks in turn.  In the odd
+// step a slot line is shared by the rows its run boundaries fall on (neighbouring blocks) and read by the planes above
+// and below (some 8 blocks on), so a run keeps most sharers on one die's L2, while all dies still stream one region.
+// Odd step, us, runs of 1 / 8 / 32 / 128 blocks: two-phase 256^3 FP64 665 / 653 / 652 / 685, 160^3 FP32 89 / 85 / 84 /
+// 88, single-phase 160^3 FP64 88 / 81 / 81 / 84 (whole eighths: 88), 125x131x119 FP32 21.7 / 20.0 / 20.0 / 20.1.  The even
+// step shares nothing but finds in its die what the odd step left there: 538 -> 524 us at 256^3, 61 -> 59 and 12.5 -> 11.7
+// us in the single-phase cases, 55 -> 50 us for ten REVs.  The grid is update_grid(blocks).
+constexpr int UPDATE_RUN = 16;
+__device__ __forceinline__ int update_block() {
     const int x = (int)blockIdx.x % NXCD, i = (int)blockIdx.x / NXCD;
-    return (i / ODD_RUN * NXCD + x) * ODD_RUN + i % ODD_RUN;
+    return (i / UPDATE_RUN * NXCD + x) * UPDATE_RUN + i % UPDATE_RUN;
 }
-inline unsigned odd_grid(long blocks) { return (unsigned)((blocks + NXCD * ODD_RUN - 1) / (NXCD * ODD_RUN) * (NXCD * ODD_RUN)); }
+inline unsigned update_grid(long blocks) {
+    return (unsigned)((blocks + NXCD * UPDATE_RUN - 1) / (NXCD * UPDATE_RUN) * (NXCD * UPDATE_RUN));
+}
 inline unsigned nblocks(long n) { return (unsigned)((n + BLOCK - 1) / BLOCK); }
 // grid of a list kernel that uses xcd_block(): per = blocks per die
 inline int xcd_per(long n) { return (int)((nblocks(n) + NXCD - 1) / NXCD); }

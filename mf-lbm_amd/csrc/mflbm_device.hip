@@ -306,7 +306,7 @@ __global__ void __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(2, 8)))
 k_collide(Dev d, CollideParams P) {
     const SlotTable& S = d.S;
-    const int m = (ODD ? odd_block() : (int)blockIdx.x) * BLOCK + (int)threadIdx.x;
+    const int m = update_block() * BLOCK + (int)threadIdx.x;
     if (m >= d.nf) return;
     const int nn = d.cpos[m];
     double cnx, cny, cnz, tf;
@@ -372,7 +372,7 @@ k_collide(Dev d, CollideParams P) {
 template <bool ODD, class C, bool STENCIL, bool STREAM>
 __global__ void __launch_bounds__(BLOCK) k_collide32(Dev d, CollideParamsDev<C> P, double gamma) {
     const SlotTable& S = d.S;
-    const int m = (ODD ? odd_block() : (int)blockIdx.x) * BLOCK + (int)threadIdx.x;
+    const int m = update_block() * BLOCK + (int)threadIdx.x;
     if (m >= d.nf) return;
     const int nn = d.cpos[m];
     C cnx, cny, cnz, tf;
@@ -2212,14 +2212,14 @@ int launch_step(mflbm_ctx* c, int ntime) {
         c->ev_used += 4;
         HIPCHK(c, hipEventRecord(ev[0], c->stream));
     }
-    const unsigned nb = nblocks(c->d.nf), nbo = odd_grid(nb);
+    const unsigned nb = update_grid(nblocks(c->d.nf));
     const bool stream = !odd && stream_even(19L * c->d.nf * (c->fp32 ? 8 : 16));
 #define MFLBM_COLLIDE32(C_, PP, STENCIL)                                                                         \
-    if (odd) LAUNCH(c, (k_collide32<true, C_, STENCIL, false>), nbo, c->d, PP, p.gamma);             \
+    if (odd) LAUNCH(c, (k_collide32<true, C_, STENCIL, false>), nb, c->d, PP, p.gamma);             \
     else if (stream) LAUNCH(c, (k_collide32<false, C_, STENCIL, true>), nb, c->d, PP, p.gamma);     \
     else LAUNCH(c, (k_collide32<false, C_, STENCIL, false>), nb, c->d, PP, p.gamma);
 #define MFLBM_COLLIDE(STENCIL)                                                                                   \
-    if (odd) LAUNCH(c, (k_collide<true, STENCIL, false>), nbo, c->d, P);                             \
+    if (odd) LAUNCH(c, (k_collide<true, STENCIL, false>), nb, c->d, P);                             \
     else if (stream) LAUNCH(c, (k_collide<false, STENCIL, true>), nb, c->d, P);                     \
     else LAUNCH(c, (k_collide<false, STENCIL, false>), nb, c->d, P);
     if (c->fp32 && c->p.precision == 2) {

@@ -36,8 +36,8 @@ constexpr int WAVE = 64;
 template <bool ODD, bool STREAM, class T, class C, int NT>
 __global__ void __launch_bounds__(NT) k_spb_collide(const SDev<T>* __restrict__ devs, const int* __restrict__ wave_sample,
                                                     const int* __restrict__ wave_first, const int* __restrict__ active,
-                                                    SPCollideParamsT<C> P, int nwaves, int per) {
-    const int w = (ODD ? odd_block() : xcd_block(per)) * (NT / WAVE) + (int)(threadIdx.x / WAVE);
+                                                    SPCollideParamsT<C> P, int nwaves) {
+    const int w = update_block() * (NT / WAVE) + (int)(threadIdx.x / WAVE);
     if (w >= nwaves) return;
     const int s = __builtin_amdgcn_readfirstlane(wave_sample[w]);
     if (!active[s]) return;
@@ -223,14 +223,12 @@ const SPCollideParamsT<float>& rates_of<float>(const mflbm_spb_ctx* c) { return 
 
 template <class T, class C, int NT>
 int launch_collide_t(mflbm_spb_ctx* c, bool odd) {
-    const long nb = ((long)c->nwaves * WAVE + NT - 1) / NT;
-    const int per = (int)((nb + NXCD - 1) / NXCD);
-    const unsigned grid = odd ? odd_grid(nb) : (unsigned)(NXCD * per);
+    const unsigned grid = update_grid(((long)c->nwaves * WAVE + NT - 1) / NT);
     if (grid == 0) return MFLBM_OK;
     const auto kern = odd ? k_spb_collide<true, false, T, C, NT>
                           : stream_even(c->pop_bytes) ? k_spb_collide<false, true, T, C, NT> : k_spb_collide<false, false, T, C, NT>;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), 0, c->stream, devs_of<T>(c), c->wave_sample, c->wave_first, c->M.active,
-                       rates_of<C>(c), c->nwaves, per);
+                       rates_of<C>(c), c->nwaves);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(c, MFLBM_ERR_HIP, "launch k_spb_collide: %s", hipGetErrorString(e));
     return MFLBM_OK;

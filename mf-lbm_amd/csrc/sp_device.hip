@@ -313,17 +313,16 @@ int sp_launch_step_t(mflbm_sp_ctx* c, int ntime, hipEvent_t* ev) {
     const Layout& L = c->L;
     const SDev<T>& d = view<T>(c);
     const bool odd = (ntime % 2) != 0;
-    const int per = xcd_per(d.nf);
-    const unsigned nbo = odd_grid(nblocks(d.nf));
+    const unsigned nb = update_grid(nblocks(d.nf));
     const bool stream = stream_even(19L * d.nf * (long)sizeof(T));
     if (c->mixed) {
-        if (odd) LAUNCH(c, (k_sp_collide<true, false, T, double>), nbo, d, c->cp, per);
-        else if (stream) LAUNCH(c, (k_sp_collide<false, true, T, double>), NXCD * per, d, c->cp, per);
-        else LAUNCH(c, (k_sp_collide<false, false, T, double>), NXCD * per, d, c->cp, per);
+        if (odd) LAUNCH(c, (k_sp_collide<true, false, T, double>), nb, d, c->cp);
+        else if (stream) LAUNCH(c, (k_sp_collide<false, true, T, double>), nb, d, c->cp);
+        else LAUNCH(c, (k_sp_collide<false, false, T, double>), nb, d, c->cp);
     } else {
-        if (odd) LAUNCH(c, (k_sp_collide<true, false, T, T>), nbo, d, rates<T>(c), per);
-        else if (stream) LAUNCH(c, (k_sp_collide<false, true, T, T>), NXCD * per, d, rates<T>(c), per);
-        else LAUNCH(c, (k_sp_collide<false, false, T, T>), NXCD * per, d, rates<T>(c), per);
+        if (odd) LAUNCH(c, (k_sp_collide<true, false, T, T>), nb, d, rates<T>(c));
+        else if (stream) LAUNCH(c, (k_sp_collide<false, true, T, T>), nb, d, rates<T>(c));
+        else LAUNCH(c, (k_sp_collide<false, false, T, T>), nb, d, rates<T>(c));
     }
     if (ev) HIPCHK(c, hipEventRecord(ev[1], c->stream));
     if (p.kper == 1 || p.jper == 1) {

@@ -119,11 +119,9 @@ __device__ __forceinline__ void sp_update_node(const SDev<T>& d, const SPCollide
     }
 }
 
-// block order of the even step: plain for FP64 storage, XCD-aware for FP32 storage (each measured the faster at 256^3, by
-// 2 %)
 template <bool ODD, bool STREAM, class T, class C>
-__global__ void __launch_bounds__(BLOCK) k_sp_collide(SDev<T> d, SPCollideParamsT<C> P, int per) {
-    const int m = (ODD ? odd_block() : sizeof(T) == sizeof(double) ? (int)blockIdx.x : xcd_block(per)) * BLOCK + (int)threadIdx.x;
+__global__ void __launch_bounds__(BLOCK) k_sp_collide(SDev<T> d, SPCollideParamsT<C> P) {
+    const int m = update_block() * BLOCK + (int)threadIdx.x;
     if (m >= d.nf) return;
     sp_update_node<ODD, STREAM, T, C>(d, P, m);
 }
