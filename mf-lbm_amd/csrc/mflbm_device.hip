@@ -47,8 +47,6 @@ struct Dev {
     // consecutive fluid nodes finds its links of one direction contiguous (index nc + wbase + rank in wave).
     SlotTable S;
     const int* map;   // padded offset -> compact index, -1 where nothing is stored
-    const int* pmap;  // padded offset -> compact index of an interior fluid node, -1 elsewhere (a folded halo node
-                      // maps to its image in map but not here: its phi is the dense one the periodic copy writes)
     const RowRec* rows;   // row records (layout.h)
     const int* cpos;  // compact index -> padded offset
     int nf;           // interior fluid nodes
@@ -62,6 +60,7 @@ struct Dev {
     // the boundary conditions read it through phi_now; the dense phi takes these values before any other reader
     // (k_phi_dense)
     double* phic;
+    unsigned pcoff;   // phic - phi in elements: both lie in one allocation, so either is one base and a 32-bit element
     // The normal field, one 32-byte record (cn_x, cn_y, cn_z, c_norm) per dense node: a neighbour's normal is one
     // cache-line access in the stencils that read it (normal extrapolation, curvature)
     double4* cn;
@@ -183,24 +182,50 @@ __device__ __forceinline__ void flag_band(const Dev& d, int b, double v) {
     if (!(fabs(v + 1.0) <= PHI_BAND)) d.notm[b] = 1;
     if (!(fabs(v - 1.0) <= PHI_BAND)) d.notp[b] = 1;
 }
-// current phi of padded node n: the compact value at a fluid node, the dense value elsewhere (one load from the
-// selected address)
-__device__ __forceinline__ double phi_now(const Dev& d, int n) {
-    const int c = d.pmap[n];
-    return *((unsigned)c < (unsigned)d.nf ? d.phic + c : d.phi + n);
+// Where the current phi of the node at ex (-1, 0, 1) of padded node n's row lies, as an element of the phi allocation:
+// the compact value of a fluid node, the dense value elsewhere (a folded halo node has its image's population slots but
+// its own dense phi).  R: the row's record at n; o: the row's own padded offset at n.
+__device__ __forceinline__ unsigned phi_slot(const Dev& d, const RowRec& R, int o, int ex) {
+    const RowRec Q{R.base, (R.bits & ROW_IMAGE) ? 0u : R.bits};
+    const unsigned c = row_rank(Q, o) + (ex < 0 ? ~0u : ex > 0 ? row_fluid(Q, o, 0) : 0u);
+    return row_fluid(Q, o, ex) ? d.pcoff + c : (unsigned)(o + ex);
 }
-// phi_now around node n, for the stencils (DENSE: the dense phi, where it is current at every node)
-template <bool DENSE = false>
-__device__ __forceinline__ double phi_at(const Dev& d, int n) {
-    return DENSE ? d.phi[n] : phi_now(d, n);
-}
+__device__ __forceinline__ double phi_now(const Dev& d, int n) { return d.phi[phi_slot(d, d.rows[n >> 4], n, 0)]; }
+// The records of the 9 rows around padded node n (entry 3 (dz + 1) + dy + 1).  One 8-byte load a row, from a table the
+// L2 holds, where a dense index map took one load a node from 64 bytes a group and two 64-bit addresses a value.  256^3
+// drainage, map / records: normals 51 / 45 us (96 / 70 registers), phi extrapolation 24 / 18, normal extrapolation 28 / 25.
+struct RowsAround {
+    RowRec r[9];
+    __device__ __forceinline__ RowsAround(const Dev& d, int n) {
+        const int g = n >> 4, sx = d.L.px >> 4, sxy = d.L.pxy >> 4;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) r[k] = d.rows[g + (k % 3 - 1) * sx + (k / 3 - 1) * sxy];
+    }
+    __device__ __forceinline__ unsigned slot(const Dev& d, int n, int ex, int ey, int ez) const {
+        return phi_slot(d, r[3 * (ez + 1) + ey + 1], n + ey * d.L.px + ez * d.L.pxy, ex);
+    }
+};
+// phi around node n for the stencils: its 18 neighbours, loaded together (DENSE: from the dense phi, where it is current
+// at every node)
 template <bool DENSE = false>
 struct PhiNowAt {
-    const Dev* d;
-    int n;
-    __device__ __forceinline__ double operator()(int a, int b, int c) const {
-        return phi_at<DENSE>(*d, n + a + b * d->L.px + c * d->L.pxy);
+    double v[19];
+    __device__ __forceinline__ PhiNowAt(const Dev& d, int n) {
+        if constexpr (DENSE) {
+#pragma unroll
+            for (int q = 1; q < 19; ++q) v[q] = d.phi[n + d.L.off(q)];
+        } else {
+            const RowsAround R(d, n);
+#pragma unroll
+            for (int q = 1; q < 19; ++q) v[q] = d.phi[R.slot(d, n, lat::EX[q], lat::EY[q], lat::EZ[q])];
+        }
     }
+    static constexpr int dir(int a, int b, int c) {
+        for (int q = 1; q < 19; ++q)
+            if (lat::EX[q] == a && lat::EY[q] == b && lat::EZ[q] == c) return q;
+        return 0;
+    }
+    __device__ __forceinline__ double operator()(int a, int b, int c) const { return v[dir(a, b, c)]; }
 };
 
 
@@ -1178,8 +1203,15 @@ __device__ __forceinline__ void phi_extrapolate_at(const Dev& d, const SolidList
     const int n = s.pos[t];
     const unsigned mk = s.mask[t];
     double v[19];
+    if constexpr (DENSE) {
 #pragma unroll
-    for (int q = 1; q < 19; ++q) v[q] = phi_at<DENSE>(d, (mk & (1u << q)) ? n + d.L.off(q) : n);
+        for (int q = 1; q < 19; ++q) v[q] = d.phi[(mk & (1u << q)) ? n + d.L.off(q) : n];
+    } else {
+        const RowsAround R(d, n);
+#pragma unroll
+        for (int q = 1; q < 19; ++q)
+            v[q] = d.phi[(mk & (1u << q)) ? R.slot(d, n, lat::EX[q], lat::EY[q], lat::EZ[q]) : (unsigned)n];
+    }
     double acc = 0.0;
 #pragma unroll
     for (int q = 1; q < 19; ++q) acc = (mk & (1u << q)) ? acc + v[q] * lat::W[q] : acc;
@@ -1292,7 +1324,7 @@ __global__ void __launch_bounds__(BLOCK) k_phi_extrapolate_b(Dev d, SolidList s,
 // the normal of node n (entry t of the normal list): stored, and whether a bit of it is set
 template <class NT, bool DENSE = false>
 __device__ __forceinline__ bool eval_normal(const Dev& d, int n, int fb, const FluidList& fl) {
-    const PhiNowAt<DENSE> P{&d, n};
+    const PhiNowAt<DENSE> P(d, n);
     double cx = dx4f(P);
     double cy = dy4f(P);
     double cz = dz4f(P);
@@ -1996,7 +2028,7 @@ struct mflbm_ctx {
     int device = 0;
     long ps = 0;                // stride of the dense arrays
     double* dense_pdf = nullptr;   // 38 dense arrays: upload/download staging, keeps never-touched slots
-    double* fields = nullptr;   // phi, the normal records (4 arrays' worth), curv, u, v, w, rho, phi_old
+    double* fields = nullptr;   // phi, compact phi, the normal records (4 arrays' worth), curv, u, v, w, rho, phi_old
     float* fields32 = nullptr;  // FP32 storage modes: the normal records in FP32
     int* role = nullptr;        // dense: fluid boundary index (>= 0) or -(extrapolation list index) - 2, else -1
     unsigned char* qbuf = nullptr;   // brick flags: notm, notp (two buffers each), bstatic, nzb, nzd, hasb
@@ -2004,7 +2036,6 @@ struct mflbm_ctx {
                                      // brick offsets of the 3 sorted lists (nbricks + 1 each), 2 sets of NWORK x NXCD
                                      // counters
     int lcap = 0;
-    double* phic = nullptr;          // compact phi (Dev::phic)
     bool phi_stale = false;          // the dense phi at fluid nodes may lag the compact phi (outside the chain's bricks)
     long nbricks = 0;
     int band_cur = 0;                // band buffers the lattice update fills until the next chain
@@ -2027,7 +2058,7 @@ struct mflbm_ctx {
     void* compact = nullptr;    // 38 population slices (compact slots + link slots), FP64 or FP32
     bool fp32 = false;          // precision 1 or 2: FP32 storage (s, a) of collide.h
     double* force = nullptr;    // 4 compact force arrays
-    int* map = nullptr;         // Dev::map, then Dev::pmap (2 x L.total)
+    int* map = nullptr;         // Dev::map
     RowRec* rows = nullptr;     // Dev::rows
     int* ibuf = nullptr;        // cpos, normal list, solid lists, fluid list positions
     int* wbuf = nullptr;        // per normal-list node: index into the fluid boundary list or -1
@@ -2332,7 +2363,7 @@ int scatter_state(mflbm_ctx* c) {
 }
 
 void free_geometry(mflbm_ctx* c) {
-    void* bufs[] = {c->compact, c->force, c->map, c->rows, c->ibuf, c->wbuf, c->mbuf, c->dbuf, c->wmask, c->wbase, c->role, c->qbuf, c->cbuf, c->phic};
+    void* bufs[] = {c->compact, c->force, c->map, c->rows, c->ibuf, c->wbuf, c->mbuf, c->dbuf, c->wmask, c->wbase, c->role, c->qbuf, c->cbuf};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     c->compact = nullptr;
@@ -2348,8 +2379,6 @@ void free_geometry(mflbm_ctx* c) {
     c->role = nullptr;
     c->qbuf = nullptr;
     c->cbuf = nullptr;
-    c->phic = nullptr;
-    c->d.phic = nullptr;
     c->have_geom = false;
     c->have_state = false;
 }
@@ -2403,14 +2432,14 @@ extern "C" int mflbm_create(const mflbm_params* prm, mflbm_ctx** out) {
         return bail(fail(c, MFLBM_ERR_HIP, "hipStreamCreate failed"));
     const long plane = (long)(L.nx + 2) * (L.ny + 2);
     if (hipMalloc(&c->dense_pdf, sizeof(double) * ps * 38) != hipSuccess ||
-        hipMalloc(&c->fields, sizeof(double) * ps * 11) != hipSuccess ||
+        hipMalloc(&c->fields, sizeof(double) * ps * 12) != hipSuccess ||
         hipMalloc(&c->walls, (size_t)ps) != hipSuccess ||
         hipMalloc(&c->planes, sizeof(double) * plane * 40) != hipSuccess ||
         hipMalloc(&c->red, sizeof(double) * (size_t)(L.nz + 1) * 32) != hipSuccess)
         return bail(fail(c, MFLBM_ERR_NOMEM, "device allocation of %.2f GB failed",
-                         (38.0 + 11.0) * 8.0 * ps / 1e9));
+                         (38.0 + 12.0) * 8.0 * ps / 1e9));
     if (hipMemset(c->dense_pdf, 0, sizeof(double) * ps * 38) != hipSuccess ||
-        hipMemset(c->fields, 0, sizeof(double) * ps * 11) != hipSuccess ||
+        hipMemset(c->fields, 0, sizeof(double) * ps * 12) != hipSuccess ||
         hipMemset(c->walls, 1, (size_t)ps) != hipSuccess || hipMemset(c->planes, 0, sizeof(double) * plane * 40) != hipSuccess)
         return bail(fail(c, MFLBM_ERR_HIP, "hipMemset failed"));
     if (c->fp32 && (hipMalloc(&c->fields32, sizeof(float) * ps * 4) != hipSuccess ||
@@ -2422,13 +2451,15 @@ extern "C" int mflbm_create(const mflbm_params* prm, mflbm_ctx** out) {
     }
     d.L = L;
     d.phi = c->fields;
-    d.cn = (double4*)(c->fields + ps);
-    d.curv = c->fields + 5 * ps;
-    c->u = c->fields + 6 * ps;
-    c->v = c->fields + 7 * ps;
-    c->w = c->fields + 8 * ps;
-    c->rho = c->fields + 9 * ps;
-    c->phi_old = c->fields + 10 * ps;
+    d.phic = c->fields + ps;   // (at most L.total fluid nodes; 2 ps elements stay below 2^32)
+    d.pcoff = (unsigned)ps;
+    d.cn = (double4*)(c->fields + 2 * ps);
+    d.curv = c->fields + 6 * ps;
+    c->u = c->fields + 7 * ps;
+    c->v = c->fields + 8 * ps;
+    c->w = c->fields + 9 * ps;
+    c->rho = c->fields + 10 * ps;
+    c->phi_old = c->fields + 11 * ps;
     d.walls = c->walls;
     d.w_in = c->planes;
     d.cphi = c->planes + plane;
@@ -2592,7 +2623,7 @@ extern "C" int mflbm_upload_geometry(mflbm_ctx* c, const int8_t* walls_h2, int32
     const size_t nd = (size_t)ns + s1w.size() + fd.size() + 1;
     HIPCHK(c, hipMalloc(&c->compact, esz * soff[19]));
     HIPCHK(c, hipMalloc(&c->force, sizeof(double) * fs * 4));
-    HIPCHK(c, hipMalloc(&c->map, 2 * sizeof(int) * L.total));   // map, then pmap
+    HIPCHK(c, hipMalloc(&c->map, sizeof(int) * L.total));
     HIPCHK(c, hipMalloc(&c->ibuf, sizeof(int) * ni));
     HIPCHK(c, hipMalloc(&c->wbuf, sizeof(int) * (wb.size() + 1)));
     if (!wb.empty()) HIPCHK(c, hipMemcpy(c->wbuf, wb.data(), sizeof(int) * wb.size(), hipMemcpyHostToDevice));
@@ -2624,11 +2655,6 @@ extern "C" int mflbm_upload_geometry(mflbm_ctx* c, const int8_t* walls_h2, int32
     hd.insert(hd.end(), fd.begin(), fd.end());
     hd.push_back(0.0);
     HIPCHK(c, hipMemcpy(c->map, cidx.data(), sizeof(int) * L.total, hipMemcpyHostToDevice));
-    {
-        std::vector<int> pm(L.total, -1);
-        for (int m = 0; m < nfl; ++m) pm[cpos[m]] = m;
-        HIPCHK(c, hipMemcpy(c->map + L.total, pm.data(), sizeof(int) * L.total, hipMemcpyHostToDevice));
-    }
     {
         std::vector<RowRec> rows;
         build_rows(L, cset, rows);
@@ -2681,8 +2707,7 @@ extern "C" int mflbm_upload_geometry(mflbm_ctx* c, const int8_t* walls_h2, int32
     HIPCHK(c, hipMemcpy(c->qbuf + 7 * nbr, hasb.data(), nbr, hipMemcpyHostToDevice));
     HIPCHK(c, hipMalloc(&c->cbuf, sizeof(int) * hc.size()));
     HIPCHK(c, hipMemcpy(c->cbuf, hc.data(), sizeof(int) * hc.size(), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMalloc(&c->phic, sizeof(double) * ((size_t)nfl + 1)));
-    HIPCHK(c, hipMemset(c->phic, 0, sizeof(double) * ((size_t)nfl + 1)));
+    HIPCHK(c, hipMemset(c->d.phic, 0, sizeof(double) * (size_t)nfl));
     c->phi_stale = false;
     c->nbricks = (long)nbr;
     c->lcap = lcap;
@@ -2702,9 +2727,7 @@ extern "C" int mflbm_upload_geometry(mflbm_ctx* c, const int8_t* walls_h2, int32
         d.S.p[19 + q] = (double*)((char*)c->compact + esz * (soff[q] + 1));
     }
     d.map = c->map;
-    d.pmap = c->map + L.total;
     d.rows = c->rows;
-    d.phic = c->phic;
     d.cpos = c->ibuf;
     d.nf = nfl;
     d.nc = nc;
