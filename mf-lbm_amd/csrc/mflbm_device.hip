@@ -165,12 +165,19 @@ __device__ __forceinline__ int plane_at(const Dev& d, int i, int j) { return i +
 constexpr int BRICK_SX = 4, BRICK_SY = 1, BRICK_SZ = 1;
 static_assert(BRICK_SX >= 1 && BRICK_SY >= 1 && BRICK_SZ >= 1 && BRICK_SX + BRICK_SY + BRICK_SZ == 6,
               "64-node bricks at least 2 nodes wide");
-__device__ __forceinline__ int brick_of(const Dev& d, int n) {
+struct Brick {
+    int x, y, z;
+};
+__device__ __forceinline__ Brick brick_at(const Dev& d, int n) {
     const int kp = n / d.L.pxy;
     const int r = n - kp * d.L.pxy;
     const int jp = r / d.L.px;
     const int ip = r - jp * d.L.px;
-    return (ip >> BRICK_SX) + d.nbx * ((jp >> BRICK_SY) + d.nby * (kp >> BRICK_SZ));
+    return Brick{ip >> BRICK_SX, jp >> BRICK_SY, kp >> BRICK_SZ};
+}
+__device__ __forceinline__ int brick_of(const Dev& d, int n) {
+    const Brick b = brick_at(d, n);
+    return b.x + d.nbx * (b.y + d.nby * b.z);
 }
 // Half-width of the band around +-1 within which phi counts as pure.  With every value of an ISO4 stencil within
 // eps of one constant, each difference is at most 2 eps and exact (Sterbenz), so |d/dx| <= (1/6 + 8/12) 2 eps and
@@ -1252,67 +1259,72 @@ __device__ __forceinline__ void wet(double& cx, double& cy, double& cz, double n
     }
 }
 // The chain stages over the bricks a plan (k_brick_plan) listed.  Each list (normal nodes, solid nodes, solid
-// nodes within one halo layer) is sorted by brick, off[b] .. off[b + 1] being brick b's entries (at most 64, the
-// nodes of a brick).  A group of G lanes takes one listed brick at a time; each group owns a contiguous run of the
-// work list (groups in the XCD-aware block order, so a die works on neighbouring bricks), and the grid is fixed:
-// the list length is known on the device only.
+// nodes within one halo layer) is sorted by brick, so the entries of the listed bricks of a row of bricks are a few
+// runs, and the plan's work items are pieces of 64 entries of a run: a wave takes an item, one entry a lane.  An item a
+// brick, 64 or 32 lanes for its up to 64 entries, left half the lanes idle and took more registers: normals, normal
+// extrapolation and phi extrapolation 24, 18 and 16 us against 16.5, 13.6 and 11.5 in a mixed-precision slug in a tube,
+// 43, 23.6 and 17 against 38, 23.6 and 15.6 in the 256^3 drainage, 8.4, 8.0 and 6.2 against 8.3, 6.8 and 4.9 in an
+// imbibition.  The grid is fixed: the list length is known on the device only.
+struct WorkItem {
+    int first;       // first entry
+    unsigned last;   // one past the last; bit 31: the bricks are quiet
+};
 struct BrickWork {
-    const int4* list;   // bricks to visit: (brick, first entry, end entry, brick quiet), NXCD sub-lists of cap items
-    const int* cnt;     // their numbers (NXCD)
+    const WorkItem* list;   // NXCD sub-lists of cap items
+    const int* cnt;         // their numbers (NXCD)
     int cap;
 };
 constexpr int CHAIN_BLOCKS = 2048;   // grid of the brick-list kernels: what the GPU holds at once (1024-8192 measured alike)
 constexpr int CHAIN_PER = CHAIN_BLOCKS / NXCD;     // work-groups per XCD
 static_assert(CHAIN_BLOCKS % NXCD == 0, "whole work-groups per XCD");
-// The work items of a group of G lanes.  A work list is kept as NXCD sub-lists (the plan appends a tile's bricks
-// to sub-list tile % NXCD, so no counter takes more than its share of the appends); the groups of XCD x take the
-// items of sub-list x in turn (work-groups are dispatched to the dies round-robin, blockIdx.x % NXCD).
-template <int G>
-struct GroupItems {
-    static constexpr int NG = BLOCK / G;
+// The work items of a wave.  A work list is kept as NXCD sub-lists (the plan appends a tile's items to sub-list
+// tile % NXCD, so no counter takes more than its share of the appends); the waves of XCD x take the items of
+// sub-list x in turn (work-groups are dispatched to the dies round-robin, blockIdx.x % NXCD).
+struct WaveItems {
+    static constexpr int STRIDE = CHAIN_PER * (BLOCK / 64);
     int i, hi, lane;
-    const int4* list;
-    __device__ __forceinline__ GroupItems(const BrickWork& w, int blk = (int)blockIdx.x) {
-        const int x = blk % NXCD;
+    const WorkItem* list;
+    WorkItem pre;
+    __device__ __forceinline__ WaveItems(const BrickWork& w) {
+        const int x = (int)blockIdx.x % NXCD;
         hi = w.cnt[x];
         list = w.list + (size_t)x * w.cap;
-        i = (blk / NXCD) * NG + (int)threadIdx.x / G;
-        lane = (int)threadIdx.x % G;
-    }
-    static constexpr int STRIDE = CHAIN_PER * NG;
-    // the item at i, with the load of the group's next item started (it overlaps this item's loads)
-    int4 pre;
-    __device__ __forceinline__ void start() {
+        i = ((int)blockIdx.x / NXCD) * (BLOCK / 64) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+        lane = (int)threadIdx.x % 64;
         if (i < hi) pre = list[i];
     }
-    __device__ __forceinline__ int4 take() {
-        const int4 it = pre;
+    // the entry of this lane in the item at i (-1: none) and whether the item is quiet; the wave's next item is
+    // loaded ahead
+    __device__ __forceinline__ int take(bool& quiet) {
+        const WorkItem it = pre;
         if (i + STRIDE < hi) pre = list[i + STRIDE];
-        return it;
+        quiet = (it.last >> 31) != 0;
+        const int t = it.first + lane;
+        return t < (int)(it.last & 0x7fffffffu) ? t : -1;
     }
 };
-// a normal of brick b has a bit set when any lane of the group says so: nzb of b and nzd of its 27-brick
-// neighbourhood (which the lattice update reads) are set.  All lanes of the wave call this together.
-template <int G>
-__device__ __forceinline__ void mark_nonzero(const Dev& d, int b, bool nz, int lane) {
-    const unsigned long long m = __ballot(nz);
-    const unsigned long long gm = G == 64 ? m : (m >> ((threadIdx.x & 63u) & ~(unsigned)(G - 1))) & ((1ull << (G & 63)) - 1ull);
-    if (!gm) return;
-    if (lane == 0) d.nzb[b] = 1;
-    const int bz = b / (d.nbx * d.nby), by = (b / d.nbx) % d.nby, bx = b % d.nbx;
-    for (int u = lane; u < 27; u += G) {
-        const int x = bx + u % 3 - 1, y = by + (u / 3) % 3 - 1, z = bz + u / 9 - 1;
-        if (x >= 0 && x < d.nbx && y >= 0 && y < d.nby && z >= 0 && z < d.nbz) d.nzd[x + d.nbx * (y + d.nby * z)] = 1;
-    }
+// Normals with a bit set (nz) at nodes n of the wave's lanes: nzb of their bricks and nzd of the 27 bricks around each
+// (which the lattice update reads) are set, brick by brick.  All lanes of the wave call this together.
+__device__ __forceinline__ void mark_nonzero(const Dev& d, int n, bool nz) {
+    unsigned long long m = __ballot(nz);
+    if (!m) return;
+    const Brick b = brick_at(d, n);
+    const int u = (int)(threadIdx.x & 63u), dx = u % 3 - 1, dy = (u / 3) % 3 - 1, dz = u / 9 - 1;
+    do {
+        const int l = __builtin_ctzll(m);
+        const int bx = __builtin_amdgcn_readlane(b.x, l), by = __builtin_amdgcn_readlane(b.y, l), bz = __builtin_amdgcn_readlane(b.z, l);
+        m &= ~__ballot(b.x == bx && b.y == by && b.z == bz);
+        const int x = bx + dx, y = by + dy, z = bz + dz;
+        if (u == 0) d.nzb[bx + d.nbx * (by + d.nby * bz)] = 1;
+        if (u < 27 && x >= 0 && x < d.nbx && y >= 0 && y < d.nby && z >= 0 && z < d.nbz) d.nzd[x + d.nbx * (y + d.nby * z)] = 1;
+    } while (m);
 }
-// lanes per brick of the two extrapolation stages (a brick has up to 64 solid entries; 16 and 64 lanes measured slower)
-constexpr int SOLID_GROUP = 32;
 // phi extrapolation at the solid nodes of the listed bricks (those whose phi an evaluated normal may read)
 __global__ void __launch_bounds__(BLOCK) k_phi_extrapolate_b(Dev d, SolidList s, BrickWork w) {
-    GroupItems<SOLID_GROUP> g(w);
-    for (g.start(); g.i < g.hi; g.i += GroupItems<SOLID_GROUP>::STRIDE) {
-        const int4 it = g.take();
-        for (int t = it.y + g.lane; t < it.z; t += SOLID_GROUP) phi_extrapolate_at(d, s, t);
+    for (WaveItems g(w); g.i < g.hi; g.i += WaveItems::STRIDE) {
+        bool quiet;
+        const int t = g.take(quiet);
+        if (t >= 0) phi_extrapolate_at(d, s, t);
     }
 }
 // interface normal and |grad phi| at the non-solid nodes of [-1, n+2]^3 (Phase_gradient.F90:33-79), with the
@@ -1372,57 +1384,38 @@ __device__ __forceinline__ bool eval_normal_extrapolate(const Dev& d, const Soli
 }
 template <class NT>
 __global__ void __launch_bounds__(BLOCK) k_normals(Dev d, NodeList nl, const int* __restrict__ wb, FluidList fl, BrickWork w) {
-    GroupItems<64> g(w);
     Rec4<NT>* const N = normals<NT>(d);
-    for (g.start(); g.i < g.hi; g.i += GroupItems<64>::STRIDE) {
-        const int4 it = g.take();
-        const int t = it.y + g.lane;
-        bool nz = false;
-        if (t < it.z) {
-            const int n = nl.pos[t];
-            if (it.w) N[n] = rec4<NT>(0.0, 0.0, 0.0, 0.0);
+    for (WaveItems g(w); g.i < g.hi; g.i += WaveItems::STRIDE) {
+        bool quiet, nz = false;
+        const int t = g.take(quiet);
+        int n = 0;
+        if (t >= 0) {
+            n = nl.pos[t];
+            if (quiet) N[n] = rec4<NT>(0.0, 0.0, 0.0, 0.0);
             else nz = eval_normal<NT>(d, n, wb[t], fl);
         }
-        mark_nonzero<64>(d, it.x, nz, g.lane);
+        mark_nonzero(d, n, nz);
     }
 }
 // normal extrapolated into the solid boundary nodes within one halo layer (Phase_gradient.F90:84-110); listed
 // bricks are evaluated, or, when q2b (every normal read is +0, so is the weighted mean), cleared
 template <class NT>
 __global__ void __launch_bounds__(BLOCK) k_normal_extrapolate(Dev d, SolidList s, BrickWork w) {
-    GroupItems<SOLID_GROUP> g(w);
     Rec4<NT>* const N = normals<NT>(d);
-    for (g.start(); g.i < g.hi; g.i += GroupItems<SOLID_GROUP>::STRIDE) {
-        const int4 it = g.take();
-        bool nz = false;
-        for (int t = it.y + g.lane; t < it.z; t += SOLID_GROUP) {
-            if (it.w) N[s.pos[t]] = rec4<NT>(0.0, 0.0, 0.0, 0.0);
-            else nz = eval_normal_extrapolate<NT>(d, s, t) || nz;
+    for (WaveItems g(w); g.i < g.hi; g.i += WaveItems::STRIDE) {
+        bool quiet, nz = false;
+        const int t = g.take(quiet);
+        int n = 0;
+        if (t >= 0) {
+            n = s.pos[t];
+            if (quiet) N[n] = rec4<NT>(0.0, 0.0, 0.0, 0.0);
+            else nz = eval_normal_extrapolate<NT>(d, s, t);
         }
-        mark_nonzero<SOLID_GROUP>(d, it.x, nz, g.lane);
+        mark_nonzero(d, n, nz);
     }
 }
 // The whole chain without brick lists (FP32 collision, whose rounding keeps phi out of the band almost everywhere):
-// one thread per entry of the normal list and of the solid list within one halo layer.  The lists are in brick
-// order, so a wave holds a few runs of entries of one brick each: the first lane of a run with a set bit sets nzd
-// of the brick's 27-brick neighbourhood (cleared before the chain).  Every lane of the wave calls this; lanes past
-// the end of the list pass b = -1 and nz = false.
-__device__ __forceinline__ void mark_nonzero_runs(const Dev& d, int b, bool nz) {
-    const unsigned long long m = __ballot(nz);
-    if (!m) return;
-    const int lane = (int)(threadIdx.x & 63u);
-    const int bp = __shfl(b, lane == 0 ? 0 : lane - 1);
-    const bool lead = lane == 0 || bp != b;
-    const unsigned long long ld = __ballot(lead);
-    const unsigned long long above = lane == 63 ? 0ull : ld & (~0ull << (lane + 1));
-    const unsigned long long run = above ? (above & (~above + 1ull)) - (1ull << lane) : ~0ull << lane;
-    if (!lead || !(m & run)) return;
-    const int bz = b / (d.nbx * d.nby), by = (b / d.nbx) % d.nby, bx = b % d.nbx;
-    for (int u = 0; u < 27; ++u) {
-        const int x = bx + u % 3 - 1, y = by + (u / 3) % 3 - 1, z = bz + u / 9 - 1;
-        if (x >= 0 && x < d.nbx && y >= 0 && y < d.nby && z >= 0 && z < d.nbz) d.nzd[x + d.nbx * (y + d.nby * z)] = 1;
-    }
-}
+// one thread per entry of the normal list and of the solid list within one halo layer; nzd is cleared before it.
 __global__ void __launch_bounds__(BLOCK) k_clear_bytes(unsigned char* p, int n) {
     const int t = (int)blockIdx.x * BLOCK + (int)threadIdx.x;
     if (t < n) p[t] = 0;
@@ -1430,25 +1423,15 @@ __global__ void __launch_bounds__(BLOCK) k_clear_bytes(unsigned char* p, int n) 
 template <class NT>
 __global__ void __launch_bounds__(BLOCK) k_normals_all(Dev d, NodeList nl, const int* __restrict__ wb, FluidList fl) {
     const int t = (int)blockIdx.x * BLOCK + (int)threadIdx.x;
-    int b = -1;
-    bool nz = false;
-    if (t < nl.n) {
-        const int n = nl.pos[t];
-        b = brick_of(d, n);
-        nz = eval_normal<NT, true>(d, n, wb[t], fl);
-    }
-    mark_nonzero_runs(d, b, nz);
+    const int n = t < nl.n ? nl.pos[t] : 0;
+    const bool nz = t < nl.n && eval_normal<NT, true>(d, n, wb[t], fl);
+    mark_nonzero(d, n, nz);
 }
 template <class NT>
 __global__ void __launch_bounds__(BLOCK) k_normal_extrapolate_all(Dev d, SolidList s) {
     const int t = (int)blockIdx.x * BLOCK + (int)threadIdx.x;
-    int b = -1;
-    bool nz = false;
-    if (t < s.n) {
-        b = brick_of(d, s.pos[t]);
-        nz = eval_normal_extrapolate<NT>(d, s, t);
-    }
-    mark_nonzero_runs(d, b, nz);
+    const bool nz = t < s.n && eval_normal_extrapolate<NT>(d, s, t);
+    mark_nonzero(d, t < s.n ? s.pos[t] : 0, nz);
 }
 // The plan of one chain.  A work-group owns TBX x TBY x TBZ bricks and stages the band flags of them and a halo
 // of two bricks in LDS.  From the band flags the lattice update left it derives q1b (every brick within one quiet
@@ -1477,7 +1460,7 @@ struct ChainPlan {
     const int* off_n;            // brick offsets of the sorted lists (nbricks + 1 each)
     const int* off_s;
     const int* off_1;
-    int4* list[NWORK];           // work lists (NXCD sub-lists of cap items each) and their counters (NXCD each)
+    WorkItem* list[NWORK];       // work lists (NXCD sub-lists of cap items each) and their counters (NXCD each)
     int cap;
     int* cnt;
     int* cnt_next;               // the counters of the next chain
@@ -1561,15 +1544,40 @@ __global__ void __launch_bounds__(BLOCK) k_brick_plan(Dev d, ChainPlan p, int fu
         take[1] = (h & 4) && (!q2 || zf);
         take[2] = (h & 2) && !q2;
     }
-    // one atomic per list and work-group (on the tile's sub-list): wave counts, the group's base, each brick's slot
+    // The runs: consecutive bricks of the row of TBX lanes that are taken with the same quiet flag.  The first lane of a
+    // run counts its items (at most one a brick: a brick has at most 64 entries, so TBX items at most).
     const int lane = (int)(threadIdx.x & 63u), wv = (int)threadIdx.x >> 6;
-    unsigned long long m[NWORK];
+    const unsigned long long row = ((1ull << TBX) - 1ull) << (lane & ~(TBX - 1)), lower = (1ull << lane) - 1ull;
+    const int* const offs[NWORK] = {p.off_n, p.off_1, p.off_s};
+    const unsigned char bit[NWORK] = {1, 4, 2}, quiet[NWORK] = {q1, q2, 0};
+    int first[NWORK], last[NWORK], items[NWORK], rank[NWORK];
 #pragma unroll
     for (int l = 0; l < NWORK; ++l) {
-        m[l] = __ballot(take[l]);
-        if (lane == 0) wcount[l][wv] = __popcll(m[l]);
+        const unsigned long long bare = __ballot(valid && !(h & bit[l]));
+        const unsigned long long loud = __ballot(take[l] && !quiet[l]), hush = __ballot(take[l] && quiet[l]);
+        const unsigned long long mine = quiet[l] ? hush : loud;
+        const unsigned long long before = ~bare & row & lower;
+        const bool lead = take[l] && !(before && (mine >> (63 - __builtin_clzll(before)) & 1ull));
+        const unsigned long long stop = ~bare & ~mine & row & ~lower;
+        const int end = stop ? __builtin_ctzll(stop) : (lane & ~(TBX - 1)) + TBX;
+        first[l] = lead ? offs[l][b] : 0;
+        last[l] = lead ? offs[l][b + end - lane] : 0;
+    }
+#pragma unroll
+    for (int l = 0; l < NWORK; ++l) {
+        items[l] = (last[l] - first[l] + 63) / 64;
+        int before = 0, total = 0;
+#pragma unroll
+        for (int k = 0; (1 << k) <= TBX; ++k) {
+            const unsigned long long m = __ballot((items[l] >> k) & 1);
+            before += __popcll(m & lower) << k;
+            total += __popcll(m) << k;
+        }
+        rank[l] = before;
+        if (lane == 0) wcount[l][wv] = total;
     }
     __syncthreads();
+    // one atomic per list and work-group, on the tile's sub-list
     const int sub = tile % NXCD;
     if (threadIdx.x < NWORK) {
         int tot = 0;
@@ -1577,14 +1585,13 @@ __global__ void __launch_bounds__(BLOCK) k_brick_plan(Dev d, ChainPlan p, int fu
         wbase[threadIdx.x] = tot ? atomicAdd(p.cnt + threadIdx.x * NXCD + sub, tot) : 0;
     }
     __syncthreads();
-    const int* const offs[NWORK] = {p.off_n, p.off_1, p.off_s};
-    const unsigned char quiet[NWORK] = {q1, q2, 0};
 #pragma unroll
     for (int l = 0; l < NWORK; ++l) {
-        if (!take[l]) continue;
-        int slot = wbase[l] + __popcll(m[l] & ((1ull << lane) - 1ull));
+        int slot = wbase[l] + rank[l];
         for (int v = 0; v < wv; ++v) slot += wcount[l][v];
-        p.list[l][(size_t)sub * p.cap + slot] = int4{b, offs[l][b], offs[l][b + 1], (int)quiet[l]};
+        WorkItem* const out = p.list[l] + (size_t)sub * p.cap + slot;
+        for (int k = 0; k < items[l]; ++k)
+            out[k] = WorkItem{first[l] + 64 * k, (unsigned)min(first[l] + 64 * k + 64, last[l]) | (quiet[l] ? 1u << 31 : 0u)};
     }
     if (tile == 0 && threadIdx.x < NWORK * NXCD) p.cnt_next[threadIdx.x] = 0;
 }
@@ -2032,7 +2039,7 @@ struct mflbm_ctx {
     float* fields32 = nullptr;  // FP32 storage modes: the normal records in FP32
     int* role = nullptr;        // dense: fluid boundary index (>= 0) or -(extrapolation list index) - 2, else -1
     unsigned char* qbuf = nullptr;   // brick flags: notm, notp (two buffers each), bstatic, nzb, nzd, hasb
-    int* cbuf = nullptr;             // chain lists: NWORK work lists (NXCD sub-lists of lcap int4 items each), the
+    int* cbuf = nullptr;             // chain lists: NWORK work lists (NXCD sub-lists of lcap items each), the
                                      // brick offsets of the 3 sorted lists (nbricks + 1 each), 2 sets of NWORK x NXCD
                                      // counters
     int lcap = 0;
@@ -2098,9 +2105,9 @@ Fold fold_of(const mflbm_params& p) {
 BrickWork brick_work(const mflbm_ctx* c, int work, int set) {
     const long nb = c->nbricks;
     const size_t lw = (size_t)NXCD * c->lcap;   // items per work list
-    const int4* lists = (const int4*)c->cbuf;
+    const WorkItem* lists = (const WorkItem*)c->cbuf;
     return BrickWork{lists + (size_t)work * lw,
-                     c->cbuf + 4 * NWORK * lw + 3 * (size_t)(nb + 1) + NXCD * (NWORK * set + work), c->lcap};
+                     c->cbuf + 2 * NWORK * lw + 3 * (size_t)(nb + 1) + NXCD * (NWORK * set + work), c->lcap};
 }
 #define CHAIN_LAUNCH(c, kern, ...)                                                                           \
     do {                                                                                                     \
@@ -2180,14 +2187,14 @@ int launch_gradient_t(mflbm_ctx* c, const FaceWork& faces) {
         p.next_p = c->qbuf + (size_t)(2 + (set ^ 1)) * nb;
         p.hasb = c->qbuf + 7 * (size_t)nb;
         const size_t lw = (size_t)NXCD * c->lcap;
-        const int* offs = c->cbuf + 4 * NWORK * lw;
+        const int* offs = c->cbuf + 2 * NWORK * lw;
         p.off_n = offs;
         p.off_s = offs + (nb + 1);
         p.off_1 = offs + 2 * (nb + 1);
-        int4* lists = (int4*)c->cbuf;
+        WorkItem* lists = (WorkItem*)c->cbuf;
         for (int l = 0; l < NWORK; ++l) p.list[l] = lists + (size_t)l * lw;
         p.cap = c->lcap;
-        int* cnts = c->cbuf + 4 * NWORK * lw + 3 * (size_t)(nb + 1);
+        int* cnts = c->cbuf + 2 * NWORK * lw + 3 * (size_t)(nb + 1);
         p.cnt = cnts + NWORK * NXCD * set;
         p.cnt_next = cnts + NWORK * NXCD * (set ^ 1);
         // no brick quiet after new geometry or state, and none with the fused chain, which does not use the flags
@@ -2687,12 +2694,12 @@ extern "C" int mflbm_upload_geometry(mflbm_ctx* c, const int8_t* walls_h2, int32
     const int ntiles = ((nbx + TBX - 1) / TBX) * ((nby + TBY - 1) / TBY) * ((nbz + TBZ - 1) / TBZ);
     const int lcap = (ntiles + NXCD - 1) / NXCD * BLOCK;   // items per sub-list: the bricks of its tiles
     const size_t lw = (size_t)NXCD * lcap;
-    std::vector<int> hc(4 * NWORK * lw + 3 * (nbr + 1) + 2 * NWORK * NXCD, 0);
+    std::vector<int> hc(2 * NWORK * lw + 3 * (nbr + 1) + 2 * NWORK * NXCD, 0);
     std::vector<unsigned char> hasb(nbr, 0);
     {
         const std::vector<int>* lists[3] = {&nrm, &spos, &s1pos};
         for (int l = 0; l < 3; ++l) {
-            int* off = hc.data() + 4 * NWORK * lw + (size_t)l * (nbr + 1);
+            int* off = hc.data() + 2 * NWORK * lw + (size_t)l * (nbr + 1);
             for (int o : *lists[l]) ++off[brick(o) + 1];
             for (size_t b = 0; b < nbr; ++b) {
                 if (off[b + 1] > 64) return fail(c, MFLBM_ERR_ARG, "brick with more than 64 chain entries");
