@@ -1434,7 +1434,9 @@ __global__ void __launch_bounds__(BLOCK) k_normal_extrapolate_all(Dev d, SolidLi
     mark_nonzero(d, t < s.n ? s.pos[t] : 0, nz);
 }
 // The plan of one chain.  A work-group owns TBX x TBY x TBZ bricks and stages the band flags of them and a halo
-// of two bricks in LDS.  From the band flags the lattice update left it derives q1b (every brick within one quiet
+// of two bricks in LDS, a row of bricks as bit masks: the 27-brick neighbourhoods are shifts and 9 words, where a byte a
+// brick took 27 LDS reads per brick and pass (256^3 drainage with its faces 37 -> 30 us,
+// 112 x 96 x 144 slug 12.4 -> 8.5, 48 x 48 x 128 tube 9.2 -> 8.3: a chain of launch, flag loads, list counters, stores).  From the band flags the lattice update left it derives q1b (every brick within one quiet
 // with one sign; no brick when `full`) over the tile and a one-brick halo, then q2b (q1b over the 27-brick
 // neighbourhood).  nzb and nzd are cleared (the chain stages set them again where they store a normal with a bit
 // set) and the next band buffers reset to bstatic.  The bricks each stage visits are appended to its work list with
@@ -1447,9 +1449,9 @@ __global__ void __launch_bounds__(BLOCK) k_normal_extrapolate_all(Dev d, SolidLi
 // read only by the chain stages after the plan, so the latency-bound face work overlaps the plan.  ntx, nty: tiles
 // per axis.
 constexpr int TBX = 8, TBY = 8, TBZ = 4;                     // TBX * TBY * TBZ == BLOCK
-constexpr int TSX = TBX + 2, TSY = TBY + 2, TSZ = TBZ + 2;   // q1b region: the tile and a one-brick halo
+constexpr int TSY = TBY + 2, TSZ = TBZ + 2;                  // rows of the q1b region: the tile and a one-brick halo
 constexpr int TUX = TBX + 4, TUY = TBY + 4, TUZ = TBZ + 4;   // band region: the tile and a two-brick halo
-static_assert(TBX * TBY * TBZ == BLOCK, "one brick per thread");
+static_assert(TBX * TBY * TBZ == BLOCK && TUX <= 16, "one brick per thread, a row of the band region in 16 lanes");
 constexpr int NWORK = 3;   // work lists: normals, normal extrapolation, phi extrapolation
 struct ChainPlan {
     const unsigned char* notm;   // band flags of the lattice update since the last chain
@@ -1467,8 +1469,9 @@ struct ChainPlan {
 };
 template <class T, int IN, int OUT, bool AFTER>
 __global__ void __launch_bounds__(BLOCK) k_brick_plan(Dev d, ChainPlan p, int full, FaceArgs a, int gface, int ntx, int nty) {
-    __shared__ unsigned char band[TUX * TUY * TUZ];
-    __shared__ unsigned char q1s[TSX * TSY * TSZ];
+    // rows of bricks as bit masks, bit x of the row: brick bx0 - 2 + x (band) or bx0 - 1 + x (quiet)
+    __shared__ unsigned band[TUY * TUZ];   // not quiet near -1 (low half) and near +1 (high half) of a brick or its x neighbours
+    __shared__ unsigned quiet1[TSY * TSZ]; // q1b (low half), and of a brick and both its x neighbours (high half)
     __shared__ int wcount[NWORK][BLOCK / 64];
     __shared__ int wbase[NWORK];
     int tile = (int)blockIdx.x;
@@ -1487,55 +1490,59 @@ __global__ void __launch_bounds__(BLOCK) k_brick_plan(Dev d, ChainPlan p, int fu
     const int b = valid ? x + d.nbx * (y + d.nby * z) : 0;
     // this brick's own flags, loaded with the staging
     const unsigned char zf = valid ? d.nzb[b] : 0, h = valid ? p.hasb[b] : 0, st = valid ? d.bstatic[b] : 0;
-    {   // every load of the staging issued before the first is used
-        constexpr int NSTAGE = (TUX * TUY * TUZ + BLOCK - 1) / BLOCK;
+    {   // 16 lanes a row of the band region; every load of the staging issued before the first is used
+        constexpr int ROWS = BLOCK / 16, NSTAGE = (TUY * TUZ + ROWS - 1) / ROWS;
+        const int xx = bx0 + (int)(threadIdx.x % 16) - 2;
         unsigned char vm[NSTAGE], vp[NSTAGE];
 #pragma unroll
         for (int k = 0; k < NSTAGE; ++k) {
-            const int t = threadIdx.x + k * BLOCK;
-            const int xx = bx0 + t % TUX - 2, yy = by0 + (t / TUX) % TUY - 2, zz = bz0 + t / (TUX * TUY) - 2;
-            const bool in = t < TUX * TUY * TUZ && inside(xx, yy, zz);
+            const int r = (int)threadIdx.x / 16 + k * ROWS;
+            const int yy = by0 + r % TUY - 2, zz = bz0 + r / TUY - 2;
+            const bool in = threadIdx.x % 16 < TUX && r < TUY * TUZ && inside(xx, yy, zz);
             const int c = in ? xx + d.nbx * (yy + d.nby * zz) : 0;
             vm[k] = in ? p.notm[c] : 0;
             vp[k] = in ? p.notp[c] : 0;
         }
 #pragma unroll
         for (int k = 0; k < NSTAGE; ++k) {
-            const int t = threadIdx.x + k * BLOCK;
-            if (t < TUX * TUY * TUZ) band[t] = (unsigned char)((vm[k] ? 1 : 0) | (vp[k] ? 2 : 0));
+            const int r = (int)threadIdx.x / 16 + k * ROWS;
+            const unsigned long long bm = __ballot(vm[k] != 0), bp = __ballot(vp[k] != 0);
+            if (threadIdx.x % 16 == 0 && r < TUY * TUZ) {
+                const int at = (int)(threadIdx.x & 63u);
+                const unsigned m = (unsigned)(bm >> at) & 0xffffu, pl = (unsigned)(bp >> at) & 0xffffu;
+                band[r] = (m | m << 1 | m >> 1) | (pl | pl << 1 | pl >> 1) << 16;
+            }
         }
     }
     __syncthreads();
-    // q1b of the region brick (lx - 1, ly - 1, lz - 1) of the tile: its neighbourhood is band (lx..lx+2, ...)
-    for (int t = threadIdx.x; t < TSX * TSY * TSZ; t += BLOCK) {
-        const int lx = t % TSX, ly = (t / TSX) % TSY, lz = t / (TSX * TSY);
-        unsigned char q = 1;   // outside the grid: quiet
-        if (inside(bx0 + lx - 1, by0 + ly - 1, bz0 + lz - 1)) {
-            unsigned char o = 0;
+    // q1b of the region row (ly - 1, lz - 1) of the tile from the 9 band rows around it; outside the grid: quiet
+    if (threadIdx.x < TSY * TSZ) {
+        const int ly = (int)threadIdx.x % TSY, lz = (int)threadIdx.x / TSY;
+        unsigned o = full != 0 ? ~0u : 0u;
 #pragma unroll
-            for (int dz = 0; dz < 3; ++dz)
+        for (int dz = 0; dz < 3; ++dz)
 #pragma unroll
-                for (int dy = 0; dy < 3; ++dy)
-#pragma unroll
-                    for (int dx = 0; dx < 3; ++dx) o |= band[(lx + dx) + TUX * ((ly + dy) + TUY * (lz + dz))];
-            const bool m = full != 0 || (o & 1), pl = full != 0 || (o & 2);
-            q = (!m || !pl) ? 1 : 0;
+            for (int dy = 0; dy < 3; ++dy) o |= band[(ly + dy) + TUY * (lz + dz)];
+        const int yy = by0 + ly - 1, zz = bz0 + lz - 1;
+        unsigned in = 0;   // bits of the row inside the grid
+        if (yy >= 0 && yy < d.nby && zz >= 0 && zz < d.nbz) {
+            in = bx0 == 0 ? ~1u : ~0u;
+            if (d.nbx - bx0 + 1 < 32) in &= (1u << (d.nbx - bx0 + 1)) - 1u;
         }
-        q1s[t] = q;
+        const unsigned q = ((~(o & (o >> 16)) >> 1) | ~in) & 0xffffu;
+        quiet1[threadIdx.x] = q | (q & (q << 1) & (q >> 1)) << 16;
     }
     __syncthreads();
     bool take[NWORK] = {false, false, false};
     unsigned char q1 = 0, q2 = 0;
     if (valid) {
-        const int r = tx + TSX * (ty + TSY * tz);   // this brick's neighbourhood corner in the q1b region
-        q1 = q1s[r + 1 + TSX * (1 + TSY)];
-        q2 = 1;
+        q1 = (unsigned char)(quiet1[ty + 1 + TSY * (tz + 1)] >> (tx + 1) & 1u);
+        unsigned q = ~0u;
 #pragma unroll
         for (int dz = 0; dz < 3; ++dz)
 #pragma unroll
-            for (int dy = 0; dy < 3; ++dy)
-#pragma unroll
-                for (int dx = 0; dx < 3; ++dx) q2 &= q1s[r + dx + TSX * (dy + TSY * dz)];
+            for (int dy = 0; dy < 3; ++dy) q &= quiet1[ty + dy + TSY * (tz + dz)];
+        q2 = (unsigned char)(q >> (17 + tx) & 1u);
         d.nzb[b] = 0;
         d.nzd[b] = 0;
         p.next_m[b] = st;   // the next lattice update adds its band flags to the static ones
