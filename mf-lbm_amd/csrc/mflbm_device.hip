@@ -639,22 +639,30 @@ __global__ void k_wrap_push_edge(Dev d) {
     copy_both<T>(d, 18, L.at(i, 1, 1), L.at(i, L.ny + 1, L.nz + 1));
 }
 // phi halo of 4 layers in the periodic directions (MPI_phi_async_pack / _sync_update, Mpi.F90:608-867):
-// each halo node of the y-z plane (x interior) takes the value of its periodic image
-__global__ void k_wrap_phi(Dev d, int wrap_y, int wrap_z) {
+// each halo node of the y-z plane (x interior) takes the value of its periodic image.  One thread a halo node: the y
+// halo's rows (8 a layer; in both directions also of the z halo's layers), then the z halo's.
+__host__ __device__ __forceinline__ long wrap_nodes(const Layout& L, int wy, int wz) {
+    return (long)L.nx * ((wy ? 8L * (wz ? L.nz + 8 : L.nz) : 0) + (wz ? 8L * L.ny : 0));
+}
+__device__ __forceinline__ void wrap_phi_at(const Dev& d, int wy, int wz, long t) {
     const Layout L = d.L;
-    const int ny8 = L.ny + 8, nz8 = L.nz + 8;
-    const long t = (long)blockIdx.x * BLOCK + threadIdx.x;
-    if (t >= (long)L.nx * ny8 * nz8) return;
-    const int i = (int)(t % L.nx) + 1;
-    const int j = (int)((t / L.nx) % ny8) - 3;
-    const int k = (int)(t / ((long)L.nx * ny8)) - 3;
-    const bool gy = j < 1 || j > L.ny, gz = k < 1 || k > L.nz;
-    if (!gy && !gz) return;
-    if (gy && !wrap_y) return;
-    if (gz && !wrap_z) return;
-    const int js = gy ? (j < 1 ? j + L.ny : j - L.ny) : j;
-    const int ks = gz ? (k < 1 ? k + L.nz : k - L.nz) : k;
+    if (t >= wrap_nodes(L, wy, wz)) return;
+    const int i = (int)(t % L.nx) + 1, yrows = wy ? 8 * (wz ? L.nz + 8 : L.nz) : 0;
+    int r = (int)(t / L.nx), j, k;
+    if (r < yrows) {
+        j = (r & 7) < 4 ? (r & 7) - 3 : L.ny + (r & 7) - 3;
+        k = (r >> 3) + (wz ? -3 : 1);
+    } else {
+        r -= yrows;
+        j = r % L.ny + 1;
+        k = r / L.ny < 4 ? r / L.ny - 3 : L.nz + r / L.ny - 3;
+    }
+    const int js = j < 1 ? j + L.ny : j > L.ny ? j - L.ny : j;
+    const int ks = k < 1 ? k + L.nz : k > L.nz ? k - L.nz : k;
     d.phi[L.at(i, j, k)] = phi_now(d, L.at(i, js, ks));
+}
+__global__ void __launch_bounds__(BLOCK) k_wrap_phi(Dev d, int wy, int wz) {
+    wrap_phi_at(d, wy, wz, (long)blockIdx.x * BLOCK + threadIdx.x);
 }
 
 // ------------------------------------------------------------------------------------------------------
@@ -1480,8 +1488,9 @@ __global__ void __launch_bounds__(BLOCK) k_normal_extrapolate_all(Dev d, SolidLi
 // of list counters is cleared for the next chain.
 // IN != 0: the first 2 gface work-groups run the inlet and outlet conditions of the step instead (k_open_faces):
 // they touch no brick flag and read interior phi through phi_now, and the phi they write in the halo planes is
-// read only by the chain stages after the plan, so the latency-bound face work overlaps the plan.  ntx, nty: tiles
-// per axis.
+// read only by the chain stages after the plan, so the latency-bound face work overlaps the plan.  The next gwrap
+// work-groups copy the periodic phi halo (wrap_phi_at), other halo nodes than the faces', likewise: its own launch took
+// 4.5 us of a 48 x 48 x 128 tube's 51 us step and 5.5 us of a 112 x 96 x 144 slug's, here it adds nothing.  ntx, nty: tiles per axis.
 constexpr int TBX = 8, TBY = 8, TBZ = 4;                     // TBX * TBY * TBZ == BLOCK
 constexpr int TSY = TBY + 2, TSZ = TBZ + 2;                  // rows of the q1b region: the tile and a one-brick halo
 constexpr int TUX = TBX + 4, TUY = TBY + 4, TUZ = TBZ + 4;   // band region: the tile and a two-brick halo
@@ -1502,7 +1511,7 @@ struct ChainPlan {
     int* cnt_next;               // the counters of the next chain
 };
 template <class T, int IN, int OUT, bool AFTER>
-__global__ void __launch_bounds__(BLOCK) k_brick_plan(Dev d, ChainPlan p, int full, FaceArgs a, int gface, int ntx, int nty) {
+__global__ void __launch_bounds__(BLOCK) k_brick_plan(Dev d, ChainPlan p, int full, FaceArgs a, int gface, int gwrap, int wy, int wz, int ntx, int nty) {
     // rows of bricks as bit masks, bit x of the row: brick bx0 - 2 + x (band) or bx0 - 1 + x (quiet)
     __shared__ unsigned band[TUY * TUZ];   // not quiet near -1 (low half) and near +1 (high half) of a brick or its x neighbours
     __shared__ unsigned quiet1[TSY * TSZ]; // q1b (low half), and of a brick and both its x neighbours (high half)
@@ -1516,6 +1525,11 @@ __global__ void __launch_bounds__(BLOCK) k_brick_plan(Dev d, ChainPlan p, int fu
         }
         tile -= 2 * gface;
     }
+    if (tile < gwrap) {
+        wrap_phi_at(d, wy, wz, (long)tile * BLOCK + threadIdx.x);
+        return;
+    }
+    tile -= gwrap;
     const int bx0 = (tile % ntx) * TBX, by0 = ((tile / ntx) % nty) * TBY, bz0 = (tile / (ntx * nty)) * TBZ;
     auto inside = [&](int x, int y, int z) { return x >= 0 && x < d.nbx && y >= 0 && y < d.nby && z >= 0 && z < d.nbz; };
     const int tx = threadIdx.x % TBX, ty = (threadIdx.x / TBX) % TBY, tz = threadIdx.x / (TBX * TBY);
@@ -2172,19 +2186,21 @@ int ensure_dense_phi(mflbm_ctx* c) {
     return MFLBM_OK;
 }
 
-// Open inlet and outlet conditions a step hands to the chain's plan launch (kind 0: none)
+// Open inlet and outlet conditions (kind 0: none) and the axes of the periodic phi halo that a step hands to the chain's
+// plan launch
 struct FaceWork {
     int in = 0, out = 0;
     bool after = false;
     FaceArgs a{};
     int gface = 0;
+    int wy = 0, wz = 0;
 };
 template <class T, int IN, int OUT, bool AFTER>
 int launch_plan_k(mflbm_ctx* c, const ChainPlan& p, int full, const FaceWork& f) {
     const int ntx = (c->d.nbx + TBX - 1) / TBX, nty = (c->d.nby + TBY - 1) / TBY, ntz = (c->d.nbz + TBZ - 1) / TBZ;
-    const int nface = IN != 0 ? 2 * f.gface : 0;
-    hipLaunchKernelGGL((k_brick_plan<T, IN, OUT, AFTER>), dim3(nface + ntx * nty * ntz), dim3(BLOCK), 0, c->stream,
-                       c->d, p, full, f.a, f.gface, ntx, nty);
+    const int nface = IN != 0 ? 2 * f.gface : 0, nwrap = (int)nblocks(wrap_nodes(c->L, f.wy, f.wz));
+    hipLaunchKernelGGL((k_brick_plan<T, IN, OUT, AFTER>), dim3(nface + nwrap + ntx * nty * ntz), dim3(BLOCK), 0,
+                       c->stream, c->d, p, full, f.a, f.gface, nwrap, f.wy, f.wz, ntx, nty);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(c, MFLBM_ERR_HIP, "launch k_brick_plan: %s", hipGetErrorString(e));
     return MFLBM_OK;
@@ -2326,9 +2342,9 @@ int launch_step(mflbm_ctx* c, int ntime) {
     return MFLBM_OK;
 }
 
-// periodic wrap and boundary conditions of one step, after the lattice update.  The combined inlet + outlet
-// condition of a domain without a porous plate is handed to the chain's plan launch through `defer` (the chain
-// follows at once), where it overlaps the plan; otherwise it is launched here.
+// periodic wrap and boundary conditions of one step, after the lattice update.  The periodic phi halo, and the combined
+// inlet + outlet condition of a domain without a porous plate, are handed to the chain's plan launch through `defer` (the
+// chain follows at once), where they overlap the plan; otherwise they are launched here.
 template <class T>
 int launch_faces(mflbm_ctx* c, bool odd, FaceWork* defer) {
     const mflbm_params& p = c->p;
@@ -2347,7 +2363,12 @@ int launch_faces(mflbm_ctx* c, bool odd, FaceWork* defer) {
             if (wy) LAUNCH(c, k_wrap_push_y<T>, nblocks((long)L.nx * L.nz), c->d);
             if (we) LAUNCH(c, k_wrap_push_edge<T>, nblocks(L.nx), c->d);
         }
-        LAUNCH(c, k_wrap_phi, nblocks((long)L.nx * (L.ny + 8) * (L.nz + 8)), c->d, p.jper, p.kper);
+        if (defer) {
+            defer->wy = p.jper;
+            defer->wz = p.kper;
+        } else {
+            LAUNCH(c, k_wrap_phi, nblocks(wrap_nodes(L, p.jper, p.kper)), c->d, p.jper, p.kper);
+        }
     }
     const unsigned gface = nblocks((long)L.nx * L.ny);
     const bool both = (p.inlet_bc == 1 || p.inlet_bc == 2) && (p.outlet_bc == 1 || p.outlet_bc == 2);
