@@ -264,7 +264,9 @@ __device__ __forceinline__ void st_pair32(double* slice, unsigned m, float s, fl
 // load every slot they touch before their first store (a load after a store through another pointer of the same
 // type must wait for it, and the slices cannot be told apart at compile time), update the registers in the order of
 // the colour-by-colour code, and store each slot once.  get/set mirror Pop<T>::at: FP64 holds (f, g); FP32 holds
-// (s, a) and a colour's value is read and written in FP64 exactly as CRef does.
+// (s, a) and a colour's value is read and written in FP64 exactly as CRef does.  In the extra work-groups of the chain's
+// plan launch too: reading and writing the slots in place there spared registers (58 for 94 of the FP64 launch, 8 waves a
+// SIMD for 5), but the plan is one short pass and the faces the longer: 256^3 drainage 31.7 / 28.5 -> 28.6 / 23.6 us.
 template <class T>
 struct SlotReg;
 template <>
@@ -303,26 +305,6 @@ struct SlotReg<float> {
         a = (float)(c ? other - x : x - other);
     }
 };
-// A slot of the velocity inlet or the convective outlet.  HOIST: held in registers (SlotReg); otherwise read and
-// written in place through Pop<T> in the same order, with fewer registers: the conditions that run in extra
-// work-groups of the chain's plan launch would otherwise lower the occupancy of the whole launch.
-template <class T, bool HOIST>
-struct FaceSlot;
-template <class T>
-struct FaceSlot<T, true> : SlotReg<T> {};
-template <class T>
-struct FaceSlot<T, false> {
-    const Dev* d;
-    int i;
-    __device__ __forceinline__ void load(const Dev& dd, int, int ii) {
-        d = &dd;
-        i = ii;
-    }
-    __device__ __forceinline__ void store(const Dev&, int, int) const {}
-    __device__ __forceinline__ double get(int c, int q) const { return (double)Pop<T>{d, c ? 19 : 0}.at(q, i); }
-    __device__ __forceinline__ void set(int c, int q, double x) const { Pop<T>{d, c ? 19 : 0}.at(q, i) = x; }
-};
-
 // The 19 slots a pressure condition reads and writes at a face node o, in registers: AFTER, the node's own; before,
 // slot q of the node at -e_q (what the next odd update pulls).  The slots of different nodes are different, so all are
 // resolved and loaded at once, both colours with one access: colour by colour and slot by slot a load waited for the
@@ -681,7 +663,7 @@ __device__ __forceinline__ void set_inlet_phi(const Dev& d, int i, int j, double
 }
 
 // inlet_bounce_back_velocity_BC_before_odd (Boundary_multiphase_inlet.F90:6-53)
-template <class T, bool HOIST = true>
+template <class T>
 __device__ __forceinline__ void bc_inlet_velocity_before(const Dev& d, int t, double phi_inlet, double sa_inject, double relaxation) {
     const Layout L = d.L;
     if (t >= L.nx * L.ny) return;
@@ -695,7 +677,7 @@ __device__ __forceinline__ void bc_inlet_velocity_before(const Dev& d, int t, do
         iw[m] = slot_index(d, QW[m], L.at(i + DI[m], j + DJ[m], 0));
         ir[m] = slot_index(d, QR[m], L.at(i, j, 1));
     }
-    FaceSlot<T, HOIST> W[5], R[5];
+    SlotReg<T> W[5], R[5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         W[m].load(d, QW[m], iw[m]);
@@ -717,7 +699,7 @@ __device__ __forceinline__ void bc_inlet_velocity_before(const Dev& d, int t, do
     for (int m = 0; m < 5; ++m) W[m].store(d, QW[m], iw[m]);
 }
 // inlet_bounce_back_velocity_BC_after_odd (Boundary_multiphase_inlet.F90:56-102)
-template <class T, bool HOIST = true>
+template <class T>
 __device__ __forceinline__ void bc_inlet_velocity_after(const Dev& d, int t, double phi_inlet, double sa_inject, double relaxation) {
     const Layout L = d.L;
     if (t >= L.nx * L.ny) return;
@@ -731,7 +713,7 @@ __device__ __forceinline__ void bc_inlet_velocity_after(const Dev& d, int t, dou
         iw[m] = slot_index(d, QW[m], o);
         ir[m] = slot_index(d, QR[m], L.at(i + DI[m], j + DJ[m], 0));
     }
-    FaceSlot<T, HOIST> W[5], R[5];
+    SlotReg<T> W[5], R[5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         W[m].load(d, QW[m], iw[m]);
@@ -820,7 +802,7 @@ __device__ __forceinline__ void bc_inlet_pressure_after(const Dev& d, int t, dou
 }
 
 // outlet_convective_BC_before_odd (Boundary_multiphase_outlet.F90:7-65)
-template <class T, bool HOIST = true>
+template <class T>
 __device__ __forceinline__ void bc_outlet_convective_before(const Dev& d, int t, double u_convec) {
     const Layout L = d.L;
     if (t >= L.nx * L.ny) return;
@@ -838,16 +820,14 @@ __device__ __forceinline__ void bc_outlet_convective_before(const Dev& d, int t,
         io[m] = slot_index(d, QS[m], L.at(i + DI[m], j + DJ[m], nz + 1));
         ii[m] = slot_index(d, QS[m], L.at(i + DI[m], j + DJ[m], nz));
     }
-    FaceSlot<T, HOIST> O[5], I[5];
+    SlotReg<T> O[5], I[5];
     double H[2][5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         O[m].load(d, QS[m], io[m]);
         I[m].load(d, QS[m], ii[m]);
-        if constexpr (HOIST) {
-            H[0][m] = d.cf[pc + QS[m] * pl];
-            H[1][m] = d.cg[pc + QS[m] * pl];
-        }
+        H[0][m] = d.cf[pc + QS[m] * pl];
+        H[1][m] = d.cg[pc + QS[m] * pl];
     }
     const double temp = 1.0 / (1.0 + u_convec);
     const int wi = d.walls[L.at(i, j, nz)];
@@ -863,10 +843,7 @@ __device__ __forceinline__ void bc_outlet_convective_before(const Dev& d, int t,
         double* hist = c == 0 ? d.cf : d.cg;
 #pragma unroll
         for (int m = 0; m < 5; ++m) {
-            double h;
-            if constexpr (HOIST) h = H[c][m];
-            else h = hist[pc + QS[m] * pl];
-            O[m].set(c, QS[m], ((h + u_convec * I[m].get(c, QS[m])) * temp) * om + O[m].get(c, QS[m]) * wd);
+            O[m].set(c, QS[m], ((H[c][m] + u_convec * I[m].get(c, QS[m])) * temp) * om + O[m].get(c, QS[m]) * wd);
         }
 #pragma unroll
         for (int m = 0; m < 5; ++m) hist[pc + QS[m] * pl] = O[m].get(c, QS[m]);
@@ -875,7 +852,7 @@ __device__ __forceinline__ void bc_outlet_convective_before(const Dev& d, int t,
     for (int m = 0; m < 5; ++m) O[m].store(d, QS[m], io[m]);
 }
 // outlet_convective_BC_after_odd (Boundary_multiphase_outlet.F90:68-127)
-template <class T, bool HOIST = true>
+template <class T>
 __device__ __forceinline__ void bc_outlet_convective_after(const Dev& d, int t, double u_convec) {
     const Layout L = d.L;
     if (t >= L.nx * L.ny) return;
@@ -893,16 +870,14 @@ __device__ __forceinline__ void bc_outlet_convective_after(const Dev& d, int t, 
         iw[m] = slot_index(d, QW[m], o);
         im[m] = slot_index(d, QW[m], om1);
     }
-    FaceSlot<T, HOIST> W[5], M[5];
+    SlotReg<T> W[5], M[5];
     double H[2][5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         W[m].load(d, QW[m], iw[m]);
         M[m].load(d, QW[m], im[m]);
-        if constexpr (HOIST) {
-            H[0][m] = d.cf[pc + QH[m] * pl];
-            H[1][m] = d.cg[pc + QH[m] * pl];
-        }
+        H[0][m] = d.cf[pc + QH[m] * pl];
+        H[1][m] = d.cg[pc + QH[m] * pl];
     }
     const double temp = 1.0 / (1.0 + u_convec);
     const int wi = d.walls[L.at(i, j, nz)];
@@ -918,10 +893,7 @@ __device__ __forceinline__ void bc_outlet_convective_after(const Dev& d, int t, 
         double* hist = c == 0 ? d.cf : d.cg;
 #pragma unroll
         for (int m = 0; m < 5; ++m) {
-            double h;
-            if constexpr (HOIST) h = H[c][m];
-            else h = hist[pc + QH[m] * pl];
-            W[m].set(c, QW[m], ((h + u_convec * M[m].get(c, QW[m])) * temp) * om + W[m].get(c, QW[m]) * wd);
+            W[m].set(c, QW[m], ((H[c][m] + u_convec * M[m].get(c, QW[m])) * temp) * om + W[m].get(c, QW[m]) * wd);
         }
 #pragma unroll
         for (int m = 0; m < 5; ++m) hist[pc + QH[m] * pl] = W[m].get(c, QW[m]);
@@ -1051,13 +1023,13 @@ __global__ void __launch_bounds__(BLOCK) k_outlet_pressure_after(Dev d, double r
 struct FaceArgs {
     double phi_inlet, sa_inject, relaxation, rho_in, u_convec, rho_out;
 };
-template <class T, int IN, int OUT, bool AFTER, bool HOIST>
+template <class T, int IN, int OUT, bool AFTER>
 __device__ __forceinline__ void open_faces_block(const Dev& d, const FaceArgs& a, int gface, int b) {
     if (b < gface) {
         const int t = b * BLOCK + (int)threadIdx.x;
         if (IN == 1) {
-            if (AFTER) bc_inlet_velocity_after<T, HOIST>(d, t, a.phi_inlet, a.sa_inject, a.relaxation);
-            else bc_inlet_velocity_before<T, HOIST>(d, t, a.phi_inlet, a.sa_inject, a.relaxation);
+            if (AFTER) bc_inlet_velocity_after<T>(d, t, a.phi_inlet, a.sa_inject, a.relaxation);
+            else bc_inlet_velocity_before<T>(d, t, a.phi_inlet, a.sa_inject, a.relaxation);
         } else {
             if (AFTER) bc_inlet_pressure_after<T>(d, t, a.phi_inlet, a.sa_inject, a.rho_in, a.relaxation);
             else bc_inlet_pressure_before<T>(d, t, a.phi_inlet, a.sa_inject, a.rho_in, a.relaxation);
@@ -1065,8 +1037,8 @@ __device__ __forceinline__ void open_faces_block(const Dev& d, const FaceArgs& a
     } else {
         const int t = (b - gface) * BLOCK + (int)threadIdx.x;
         if (OUT == 1) {
-            if (AFTER) bc_outlet_convective_after<T, HOIST>(d, t, a.u_convec);
-            else bc_outlet_convective_before<T, HOIST>(d, t, a.u_convec);
+            if (AFTER) bc_outlet_convective_after<T>(d, t, a.u_convec);
+            else bc_outlet_convective_before<T>(d, t, a.u_convec);
         } else {
             if (AFTER) bc_outlet_pressure_after<T>(d, t, a.rho_out);
             else bc_outlet_pressure_before<T>(d, t, a.rho_out);
@@ -1075,7 +1047,7 @@ __device__ __forceinline__ void open_faces_block(const Dev& d, const FaceArgs& a
 }
 template <class T, int IN, int OUT, bool AFTER>
 __global__ void __launch_bounds__(BLOCK) k_open_faces(Dev d, FaceArgs a, int gface) {
-    open_faces_block<T, IN, OUT, AFTER, true>(d, a, gface, (int)blockIdx.x);
+    open_faces_block<T, IN, OUT, AFTER>(d, a, gface, (int)blockIdx.x);
 }
 
 // porous_plate_BC_before_odd / _after_odd (Boundary_multiphase_other.F90:8-184); `blocked` is the colour
@@ -1520,7 +1492,7 @@ __global__ void __launch_bounds__(BLOCK) k_brick_plan(Dev d, ChainPlan p, int fu
     int tile = (int)blockIdx.x;
     if (IN != 0) {
         if (tile < 2 * gface) {
-            open_faces_block<T, IN, OUT, AFTER, false>(d, a, gface, tile);
+            open_faces_block<T, IN, OUT, AFTER>(d, a, gface, tile);
             return;
         }
         tile -= 2 * gface;
