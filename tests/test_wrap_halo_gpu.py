@@ -1,6 +1,7 @@
-"""The periodic phi halo is copied one thread a halo node inside the chain's plan launch (MFLBM_CHAIN=all: in its own):
-y, z and both directions periodic, and y periodic between an open inlet and outlet, odd sizes with partial work-groups, an
-interface across the periodic faces: phi, its halo and every population bit for bit against the oracle."""
+"""The periodic phi halo is copied one thread a halo node inside the chain's first launch (the plan's, or with
+MFLBM_CHAIN=all the whole-list one): y, z and both directions periodic, and y periodic between an open inlet and outlet,
+odd sizes with partial work-groups, an interface near the periodic faces: phi, its halo and every population bit for bit
+against the oracle."""
 import numpy as np
 import pytest
 
