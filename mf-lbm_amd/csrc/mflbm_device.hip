@@ -159,7 +159,7 @@ __device__ __forceinline__ Pop<T> gpop(const Dev& d) { return Pop<T>{&d, 19}; }
 __device__ __forceinline__ int plane_at(const Dev& d, int i, int j) { return i + j * (d.L.nx + 2); }
 
 // brick of padded offset n: 2^BRICK_SX x 2^BRICK_SY x 2^BRICK_SZ padded nodes (16 x 2 x 2: a brick's rows are
-// whole 128-byte lines of a dense FP64 field, so the chain stages that take one brick per wave touch few lines
+// whole 128-byte lines of a dense FP64 field, so the chain stages, which take runs of bricks of a row, touch few lines
 // per access).  The brick flags need every brick at least 2 nodes wide in each axis (a normal depends on phi
 // within 2 nodes: its stencil and the fluid neighbours of the stencil's solid nodes).
 constexpr int BRICK_SX = 4, BRICK_SY = 1, BRICK_SZ = 1;
