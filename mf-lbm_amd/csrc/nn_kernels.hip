@@ -10,6 +10,7 @@
 // kernel flipped and its channel roles swapped (mflbm_nn_weights_to_bf16 writes both forms).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 
@@ -743,6 +744,25 @@ extern "C" int mflbm_nn_mfma_probe(const void* a, const void* b, float* d, void*
     return launched((hipStream_t)stream);
 }
 
+namespace {
+// Estimated us of the two forward kernels: the latency of a work-group, which grows with the input channels, or, with more
+// work-groups than are in flight at once, so many times it.  Within 25 % of the times measured over d, h, w from 1 to 256.
+// k_conv_fwd: 128 positions x 32 channels a work-group; along an axis one node long a third of the offsets is inside,
+// and a wave skips the loads of the others.
+double untiled_us(const Shape& S, int cin, int cout) {
+    const double thin = (S.d == 1 ? 1.0 / 3 : 1.0) * (S.h == 1 ? 1.0 / 3 : 1.0) * (S.w == 1 ? 1.0 / 3 : 1.0);
+    const double groups = (double)((S.count() + 127) / 128) * ((cout + 31) / 32), in_flight = cin >= 64 ? 330 : cin >= 32 ? 560 : 800;
+    return (4.0 + 0.45 * cin) * std::max(0.7 + 0.3 * thin, (0.5 + 0.5 * thin) * groups / in_flight);
+}
+// k_conv_tile: whole tiles, however much of them lies in the domain; per: us of a work-group per input channel
+template <int MT, int NCO, int WP, int WC, int TZ, int TY, int TX, int KG>
+double tile_us(const Shape& S, int cin, int cout, double per, double in_flight) {
+    using T = ConvTile<MT, NCO, WP, WC, TZ, TY, TX, KG>;
+    const double groups = (double)S.n * ((S.d + TZ - 1) / TZ) * ((S.h + TY - 1) / TY) * ((S.w + TX - 1) / TX) * ((cout + T::CO - 1) / T::CO);
+    return (4.0 + per * cin) * std::max(1.0, groups / in_flight);
+}
+}  // namespace
+
 extern "C" int mflbm_nn_conv3d_fwd(const void* x, const void* wf, const float* bias, void* y, int32_t n, int32_t d,
                                    int32_t h, int32_t w, int32_t cin, int32_t cout, int32_t relu, void* stream) {
     if (!x || !wf || !y || n < 1 || d < 1 || h < 1 || w < 1 || cin < 8 || cin % 8 || cout < 1) return MFLBM_ERR_ARG;
@@ -750,26 +770,39 @@ extern "C" int mflbm_nn_conv3d_fwd(const void* x, const void* wf, const float* b
     const long M = S.count();
     hipStream_t st = (hipStream_t)stream;
     const int kp = kpad_of(cin);
-    // Tile by channels (what fits 160 KB of LDS with the whole cin) and by the number of work-groups: the large tiles
-    // read less halo and fewer fragments per product, but need 256 work-groups to use every compute unit.  Without the
-    // tile (more than 256 input channels, or planes beyond a 2 GiB window): k_conv_fwd.
+    // Tile by channels (the tile of all cin channels, up to 256 of them, in the 160 KB of LDS) and by the number of
+    // work-groups: the large tiles read less halo and fewer fragments per product, but need 256 work-groups to use every
+    // compute unit.  Without the tile: more than 256 input channels, planes beyond a 2 GiB window, and domains that fill so
+    // little of their tiles that the whole tiles would take longer than k_conv_fwd, which pays for no position outside the
+    // domain.  us tiled / untiled: 1 x 1 x 256 x 256 32 -> 32 29 / 18, 256 -> 256 3491 / 1017, 4 x 1 x 64 x 64 64 -> 64
+    // 39 / 27, 512 x 1 x 1 x 1 64 -> 64 71 / 25, 8 x 9^3 256 -> 256 219 / 182; but 16 x 1 x 1 x 64 64 -> 64 20 / 25, 4 x 4^3
+    // 256 -> 256 56 / 118, 4 x 64 x 3 x 16 128 -> 128 34 / 89.
     if (cin <= 256 && 10L * h * w * cin * 2 < (1L << 31) && (long)cout * kp * 2 < (1L << 31)) {
+        const double tu = untiled_us(S, cin, cout);
         const long tiles8 = (long)n * ((d + 7) / 8) * ((h + 7) / 8) * ((w + 7) / 8);   // 8 x 8 x 8 tiles
-#define TILE(...) launch_conv_tile<__VA_ARGS__>(x, wf, bias, y, S, (int)cin, (int)cout, kp, (int)relu, st)
-        // fragments of positions and of channels, waves along positions and channels, tile, steps per weight stage
+        // PER, FLIGHT: tile_us; then fragments of positions and of channels, waves along positions and channels, tile, steps
+        // per weight stage
+#define TILE_US(PER, FLIGHT, ...) tile_us<__VA_ARGS__>(S, cin, cout, PER, FLIGHT)
+#define TILE(PER, FLIGHT, ...) \
+    if (TILE_US(PER, FLIGHT, __VA_ARGS__) <= tu) return launch_conv_tile<__VA_ARGS__>(x, wf, bias, y, S, (int)cin, (int)cout, kp, (int)relu, st)
+#define TILES(BIG, SMALL) \
+    if (tiles8 * ((cout + 63) / 64) >= 256 && TILE_US BIG <= TILE_US SMALL) { TILE BIG; } else { TILE SMALL; }
         if (cin <= 32) {   // 4 x 64^3, us before / after: 8 -> 32 75 / 44, 32 -> 8 196 / 85, 32 -> 32 254 / 116, 32 -> 64 483 / 175
-            if (cout <= 16) return TILE(2, 1, 8, 1, 4, 8, 8, 8);
-            if (cout > 32) return TILE(4, 4, 4, 1, 4, 8, 8, 1);
-            if (cin <= 16) return TILE(4, 2, 4, 1, 4, 8, 8, 4);
-            return TILE(2, 2, 8, 1, 4, 8, 8, 4);
+            if (cout <= 16) { TILE(0.15, 400, 2, 1, 8, 1, 4, 8, 8, 8); }
+            else if (cout > 32) { TILE(0.36, 400, 4, 4, 4, 1, 4, 8, 8, 1); }
+            else if (cin <= 16) { TILE(0.19, 400, 4, 2, 4, 1, 4, 8, 8, 4); }
+            else { TILE(0.22, 390, 2, 2, 8, 1, 4, 8, 8, 4); }
+        } else if (cin <= 64) {   // 4 x 64^3 64 -> 32 782 / 204; 4 x 32^3 64 -> 64 206 / 46 (61 in the small tile); 4 x 16^3 64 -> 128 52 / 23 (40 in the large)
+            if (cout <= 32) { TILES((0.33, 256, 4, 2, 8, 1, 8, 8, 8, 4), (0.24, 256, 2, 2, 8, 1, 4, 8, 8, 4)) }
+            else { TILES((0.55, 256, 4, 4, 8, 1, 8, 8, 8, 2), (0.25, 256, 2, 2, 4, 2, 4, 4, 8, 4)) }
+        } else if (cin <= 128) {   // 4 x 16^3 128 -> 128 100 / 36, 4 x 32^3 128 -> 64 400 / 139
+            TILE(0.22, 256, 2, 2, 4, 2, 4, 4, 8, 8);
+        } else {   // 4 x 8^3 256 -> 256 125 / 57, 4 x 16^3 256 -> 128 195 / 118
+            TILE(0.2, 256, 1, 2, 4, 2, 4, 4, 4, 4);
         }
-        if (cin <= 64) {   // 4 x 64^3 64 -> 32 782 / 204; 4 x 32^3 64 -> 64 206 / 46 (61 in the small tile); 4 x 16^3 64 -> 128 52 / 23 (40 in the large)
-            if (cout <= 32) return tiles8 >= 256 ? TILE(4, 2, 8, 1, 8, 8, 8, 4) : TILE(2, 2, 8, 1, 4, 8, 8, 4);
-            return tiles8 * ((cout + 63) / 64) >= 256 ? TILE(4, 4, 8, 1, 8, 8, 8, 2) : TILE(2, 2, 4, 2, 4, 4, 8, 4);
-        }
-        if (cin <= 128) return TILE(2, 2, 4, 2, 4, 4, 8, 8);   // 4 x 16^3 128 -> 128 100 / 36, 4 x 32^3 128 -> 64 400 / 139
-        return TILE(1, 2, 4, 2, 4, 4, 4, 4);                   // 4 x 8^3 256 -> 256 125 / 57, 4 x 16^3 256 -> 128 195 / 118
+#undef TILES
 #undef TILE
+#undef TILE_US
     }
     const dim3 grid((unsigned)((M + 127) / 128), (unsigned)((cout + 31) / 32));
     if (relu)
