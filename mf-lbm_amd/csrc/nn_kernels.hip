@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <mutex>
 
@@ -350,7 +351,7 @@ __host__ __device__ inline long dw_window(const Shape& S, int cin, long chunk) {
 template <bool ORDERED, int NC, bool FAR>
 __global__ void __launch_bounds__(NT, 2) k_conv_dw(const __bf16* __restrict__ x, const __bf16* __restrict__ dy,
                                                    float* __restrict__ dw, Shape S, int cin, int cout, long chunk,
-                                                   int nco, int nci, int total) {
+                                                   int nco, int nci, int total, int zfirst) {
     __shared__ __attribute__((aligned(16))) __bf16 xs[2][DW_ROWS][16];
     __shared__ __attribute__((aligned(16))) __bf16 ys[2][NC][32][16];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -358,7 +359,7 @@ __global__ void __launch_bounds__(NT, 2) k_conv_dw(const __bf16* __restrict__ x,
     // each die takes a run of consecutive chunks, all channel groups of one next to each other: they share its L2
     const int g = (int)(blockIdx.x % NXCD) * (int)(gridDim.x / NXCD) + (int)(blockIdx.x / NXCD);
     if (g >= total) return;
-    const int zc = g / (nco * nci);
+    const int zc = zfirst + g / (nco * nci);
     const int co0 = (g % nco) * (16 * NC);
     const int ci0 = (g / nco % nci) * 16;
     const int K = 27 * cin;
@@ -499,10 +500,15 @@ void launch_conv_dw(const void* x, const void* dy, float* dw, const Shape& S, in
     const int nc = cout > 16 && (cout + 31) / 32 * ny * nz >= 256 ? 2 : 1;
     const bool far = dw_window(S, cin, chunk) >= (1L << 31) || chunk * cout * 2 >= (1L << 31);
     const auto kern = far ? k_conv_dw<ORDERED, 1, true> : nc == 2 ? k_conv_dw<ORDERED, 2, false> : k_conv_dw<ORDERED, 1, false>;
-    const int nco = (cout + 16 * (far ? 1 : nc) - 1) / (16 * (far ? 1 : nc));
-    const long total = nco * ny * nz;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((total + NXCD - 1) / NXCD * NXCD)), dim3(NT), 0, st, (const __bf16*)x,
-                       (const __bf16*)dy, dw, S, cin, cout, chunk, nco, (int)ny, (int)total);
+    const long nco = (cout + 16 * (far ? 1 : nc) - 1) / (16 * (far ? 1 : nc));
+    // a launch has less than 2^32 threads: beyond 2^24 work-groups the chunks take several (any weight matrix that fits the
+    // memory has fewer than 2^24 channel groups)
+    const long zper = std::max(1L, ((1L << 24) - NXCD) / (nco * ny));
+    for (long z0 = 0; z0 < nz; z0 += zper) {
+        const long total = nco * ny * std::min(zper, nz - z0);
+        hipLaunchKernelGGL(kern, dim3((unsigned)((total + NXCD - 1) / NXCD * NXCD)), dim3(NT), 0, st, (const __bf16*)x,
+                           (const __bf16*)dy, dw, S, cin, cout, chunk, (int)nco, (int)ny, (int)total, (int)z0);
+    }
 }
 
 // positions per chunk of the weight- and bias-gradient sums
@@ -759,6 +765,7 @@ template <int MT, int NCO, int WP, int WC, int TZ, int TY, int TX, int KG>
 double tile_us(const Shape& S, int cin, int cout, double per, double in_flight) {
     using T = ConvTile<MT, NCO, WP, WC, TZ, TY, TX, KG>;
     const double groups = (double)S.n * ((S.d + TZ - 1) / TZ) * ((S.h + TY - 1) / TY) * ((S.w + TX - 1) / TX) * ((cout + T::CO - 1) / T::CO);
+    if ((groups + NXCD) * T::THREADS >= 4294967296.0) return HUGE_VAL;   // a launch has less than 2^32 threads
     return (4.0 + per * cin) * std::max(1.0, groups / in_flight);
 }
 }  // namespace
