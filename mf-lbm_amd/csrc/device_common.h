@@ -102,7 +102,8 @@ __device__ __forceinline__ void odd_neighbour_slots(const RowRec* rows_, const L
     }
 }
 
-// Whether the even step of a state of these bytes (fluid nodes only) reads and writes its slots non-temporally.  The
+// Whether the even step of a state of these bytes (fluid nodes only; of a batch, those of the samples still running)
+// reads and writes its slots non-temporally.  The
 // even step touches every slot line once, whole: beyond what the 256 MB last-level cache keeps from step to step its
 // lines only push out those that are read again (the odd step's shared lines, normals, phi, row records).  us per step
 // (even and odd mean), cached / streamed: two-phase FP64 90 MB 71 / 77, 196 MB 137 / 130, 362 MB 247 / 211, 1349 MB

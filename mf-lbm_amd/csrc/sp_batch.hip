@@ -177,7 +177,7 @@ struct mflbm_spb_ctx {
     std::vector<SDev<float>> dev32;
     int nwaves = 0;
     long nfluid = 0;
-    long pop_bytes = 0;                  // populations of the fluid nodes of all samples
+    long running_bytes = 0;              // populations of the fluid nodes of the samples still running (stream_even)
     hipStream_t stream = nullptr;
     void* pop = nullptr;                 // all samples' population slices
     std::vector<void*> bufs;             // maps, cpos, link masks and bases of every sample
@@ -192,12 +192,13 @@ struct mflbm_spb_ctx {
     Monitor M{};
     int* mon_int = nullptr;              // active, conv_step, period, nactive
     double* mon_dbl = nullptr;           // q_prev, q_last
-    int* nactive_h = nullptr;            // pinned
+    int* mon_h = nullptr;                // pinned copy of mon_int
     double* staging = nullptr;           // dense upload/download buffer (19 arrays of the largest sample)
     long staging_len = 0;
     Downloader dl;                       // pinned ring of the downloads
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
+    // one monitor period, with cached and with streamed even steps; each is captured when it is first needed
+    hipGraph_t graph[2] = {};
+    hipGraphExec_t graph_exec[2] = {};
     bool committed = false;
     std::string err;
 };
@@ -226,7 +227,7 @@ int launch_collide_t(mflbm_spb_ctx* c, bool odd) {
     const unsigned grid = update_grid(((long)c->nwaves * WAVE + NT - 1) / NT);
     if (grid == 0) return MFLBM_OK;
     const auto kern = odd ? k_spb_collide<true, false, T, C, NT>
-                          : stream_even(c->pop_bytes) ? k_spb_collide<false, true, T, C, NT> : k_spb_collide<false, false, T, C, NT>;
+                          : stream_even(c->running_bytes) ? k_spb_collide<false, true, T, C, NT> : k_spb_collide<false, false, T, C, NT>;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), 0, c->stream, devs_of<T>(c), c->wave_sample, c->wave_first, c->M.active,
                        rates_of<C>(c), c->nwaves);
     const hipError_t e = hipGetLastError();
@@ -308,10 +309,12 @@ int period(mflbm_spb_ctx* c) {
 }
 
 void free_all(mflbm_spb_ctx* c) {
-    if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
-    if (c->graph) (void)hipGraphDestroy(c->graph);
-    c->graph_exec = nullptr;
-    c->graph = nullptr;
+    for (int k = 0; k < 2; ++k) {
+        if (c->graph_exec[k]) (void)hipGraphExecDestroy(c->graph_exec[k]);
+        if (c->graph[k]) (void)hipGraphDestroy(c->graph[k]);
+        c->graph_exec[k] = nullptr;
+        c->graph[k] = nullptr;
+    }
     for (void* b : c->bufs)
         if (b) (void)hipFree(b);
     c->bufs.clear();
@@ -319,9 +322,9 @@ void free_all(mflbm_spb_ctx* c) {
                    c->mon_int, c->mon_dbl, c->staging};
     for (void* b : own)
         if (b) (void)hipFree(b);
-    if (c->nactive_h) (void)hipHostFree(c->nactive_h);
+    if (c->mon_h) (void)hipHostFree(c->mon_h);
     c->pop = c->devs = nullptr;
-    c->wave_sample = c->wave_first = c->nwave = c->nzs = c->yper = c->mon_int = c->nactive_h = nullptr;
+    c->wave_sample = c->wave_first = c->nwave = c->nzs = c->yper = c->mon_int = c->mon_h = nullptr;
     c->wave_sum = c->mon_dbl = c->staging = nullptr;
 }
 
@@ -340,6 +343,8 @@ int init_state_t(mflbm_spb_ctx* c) {
     return MFLBM_OK;
 }
 
+long fluid_bytes(const mflbm_spb_ctx* c, int s) { return 19L * (c->fp32 ? 4 : 8) * c->nf[s]; }
+
 int reset_monitor(mflbm_spb_ctx* c) {
     const int n = (int)c->host.size();
     LAUNCH(c, k_spb_set_int, nblocks(n), c->M.active, n, 1);
@@ -347,6 +352,8 @@ int reset_monitor(mflbm_spb_ctx* c) {
     LAUNCH(c, k_spb_set_int, 1u, c->M.period, 1, 0);
     LAUNCH(c, k_spb_fill<double>, nblocks(2L * n), c->mon_dbl, 2L * n, 0.0);
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->running_bytes = 0;
+    for (int s = 0; s < n; ++s) c->running_bytes += fluid_bytes(c, s);
     return MFLBM_OK;
 }
 
@@ -443,7 +450,6 @@ extern "C" int mflbm_spb_commit(mflbm_spb_ctx* c) {
     c->nfluid = P.nfluid;
     c->nwaves = P.nwaves;
     const long elems = P.elems, maxdense = P.maxdense;
-    c->pop_bytes = 19L * esz * P.nfluid;
     const int waves = P.nwaves;
     // device buffers
     HIPCHK(c, hipMalloc(&c->pop, (size_t)(esz * std::max(elems, 1L))));
@@ -520,7 +526,7 @@ extern "C" int mflbm_spb_commit(mflbm_spb_ctx* c) {
     HIPCHK(c, hipMalloc(&c->wave_sum, sizeof(double) * ws.size()));
     HIPCHK(c, hipMalloc(&c->mon_int, sizeof(int) * (3 * (size_t)n + 2)));
     HIPCHK(c, hipMalloc(&c->mon_dbl, sizeof(double) * 2 * (size_t)n));
-    HIPCHK(c, hipHostMalloc((void**)&c->nactive_h, sizeof(int)));
+    HIPCHK(c, hipHostMalloc((void**)&c->mon_h, sizeof(int) * (3 * (size_t)n + 2)));
     HIPCHK(c, hipMemcpy(c->wave_sample, ws.data(), sizeof(int) * ws.size(), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->wave_first, c->wave_first_h.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->nwave, c->nwave_h.data(), sizeof(int) * n, hipMemcpyHostToDevice));
@@ -672,26 +678,30 @@ extern "C" int mflbm_spb_run_steady(mflbm_spb_ctx* c, int32_t max_periods, int32
     if (!c) return MFLBM_ERR_ARG;
     if (!c->committed) return fail(c, MFLBM_ERR_STATE, "not committed");
     if (max_periods < 0) return fail(c, MFLBM_ERR_ARG, "max_periods < 0");
-    if (!c->graph_exec) {
-        HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        const int rc = period(c);
-        hipGraph_t g = nullptr;
-        const hipError_t e = hipStreamEndCapture(c->stream, &g);
-        if (rc) {
-            if (g) (void)hipGraphDestroy(g);
-            return rc;
-        }
-        if (e != hipSuccess) return fail(c, MFLBM_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
-        c->graph = g;
-        HIPCHK(c, hipGraphInstantiate(&c->graph_exec, c->graph, nullptr, nullptr, 0));
-    }
+    const size_t n = c->host.size();
     int left = 1;
     for (int k = 0; k < max_periods; ++k) {
-        HIPCHK(c, hipGraphLaunch(c->graph_exec, c->stream));
-        HIPCHK(c, hipMemcpyAsync(c->nactive_h, c->mon_int + 3 * c->host.size(), sizeof(int), hipMemcpyDeviceToHost,
-                                 c->stream));
+        const int v = stream_even(c->running_bytes) ? 1 : 0;
+        if (!c->graph_exec[v]) {
+            HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+            const int rc = period(c);
+            hipGraph_t g = nullptr;
+            const hipError_t e = hipStreamEndCapture(c->stream, &g);
+            if (rc) {
+                if (g) (void)hipGraphDestroy(g);
+                return rc;
+            }
+            if (e != hipSuccess) return fail(c, MFLBM_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
+            c->graph[v] = g;
+            HIPCHK(c, hipGraphInstantiate(&c->graph_exec[v], g, nullptr, nullptr, 0));
+        }
+        HIPCHK(c, hipGraphLaunch(c->graph_exec[v], c->stream));
+        HIPCHK(c, hipMemcpyAsync(c->mon_h, c->mon_int, sizeof(int) * (3 * n + 1), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        left = *c->nactive_h;
+        c->running_bytes = 0;
+        for (size_t s = 0; s < n; ++s)
+            if (c->mon_h[s]) c->running_bytes += fluid_bytes(c, (int)s);
+        left = c->mon_h[3 * n];
         if (left == 0) break;
     }
     if (nactive) *nactive = left;
