@@ -1433,11 +1433,37 @@ __global__ void __launch_bounds__(BLOCK) k_normals_all(Dev d, NodeList nl, const
     const bool nz = t < nl.n && eval_normal<NT, true>(d, n, wb[t], fl);
     mark_nonzero(d, n, nz);
 }
+// The same marking for a wave of entries of the solid list, which holds few entries a brick, so a wave spans many: the
+// bricks' runs side by side, the first lane of a run with a set bit setting the flags (brick by brick took the kernel from
+// 102 to 111 us at 256^3 FP32 and from 8.7 to 11.2 at 96^3; the normals' waves span one to three bricks and are
+// faster brick by brick, 87 against 90 and 7.5 against 9.6).  Every lane of the wave calls this; lanes past the end of the list
+// pass b = -1 and nz = false.
+__device__ __forceinline__ void mark_nonzero_runs(const Dev& d, int b, bool nz) {
+    const unsigned long long m = __ballot(nz);
+    if (!m) return;
+    const int lane = (int)(threadIdx.x & 63u);
+    const int bp = __shfl(b, lane == 0 ? 0 : lane - 1);
+    const bool lead = lane == 0 || bp != b;
+    const unsigned long long ld = __ballot(lead);
+    const unsigned long long above = lane == 63 ? 0ull : ld & (~0ull << (lane + 1));
+    const unsigned long long run = above ? (above & (~above + 1ull)) - (1ull << lane) : ~0ull << lane;
+    if (!lead || !(m & run)) return;
+    const int bz = b / (d.nbx * d.nby), by = (b / d.nbx) % d.nby, bx = b % d.nbx;
+    for (int u = 0; u < 27; ++u) {
+        const int x = bx + u % 3 - 1, y = by + (u / 3) % 3 - 1, z = bz + u / 9 - 1;
+        if (x >= 0 && x < d.nbx && y >= 0 && y < d.nby && z >= 0 && z < d.nbz) d.nzd[x + d.nbx * (y + d.nby * z)] = 1;
+    }
+}
 template <class NT>
 __global__ void __launch_bounds__(BLOCK) k_normal_extrapolate_all(Dev d, SolidList s) {
     const int t = (int)blockIdx.x * BLOCK + (int)threadIdx.x;
-    const bool nz = t < s.n && eval_normal_extrapolate<NT>(d, s, t);
-    mark_nonzero(d, t < s.n ? s.pos[t] : 0, nz);
+    int b = -1;
+    bool nz = false;
+    if (t < s.n) {
+        b = brick_of(d, s.pos[t]);
+        nz = eval_normal_extrapolate<NT>(d, s, t);
+    }
+    mark_nonzero_runs(d, b, nz);
 }
 // The plan of one chain.  A work-group owns TBX x TBY x TBZ bricks and stages the band flags of them and a halo
 // of two bricks in LDS, a row of bricks as bit masks: the 27-brick neighbourhoods are shifts and 9 words, where a byte a
