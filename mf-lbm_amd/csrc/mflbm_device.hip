@@ -212,20 +212,14 @@ struct RowsAround {
         return phi_slot(d, r[3 * (ez + 1) + ey + 1], n + ey * d.L.px + ez * d.L.pxy, ex);
     }
 };
-// phi around node n for the stencils: its 18 neighbours, loaded together (DENSE: from the dense phi, where it is current
-// at every node)
+// phi around node n for the stencils, from the row records: its 18 neighbours, loaded together
 template <bool DENSE = false>
 struct PhiNowAt {
     double v[19];
     __device__ __forceinline__ PhiNowAt(const Dev& d, int n) {
-        if constexpr (DENSE) {
+        const RowsAround R(d, n);
 #pragma unroll
-            for (int q = 1; q < 19; ++q) v[q] = d.phi[n + d.L.off(q)];
-        } else {
-            const RowsAround R(d, n);
-#pragma unroll
-            for (int q = 1; q < 19; ++q) v[q] = d.phi[R.slot(d, n, lat::EX[q], lat::EY[q], lat::EZ[q])];
-        }
+        for (int q = 1; q < 19; ++q) v[q] = d.phi[R.slot(d, n, lat::EX[q], lat::EY[q], lat::EZ[q])];
     }
     static constexpr int dir(int a, int b, int c) {
         for (int q = 1; q < 19; ++q)
@@ -233,6 +227,15 @@ struct PhiNowAt {
         return 0;
     }
     __device__ __forceinline__ double operator()(int a, int b, int c) const { return v[dir(a, b, c)]; }
+};
+// DENSE: from the dense phi, where it is current at every node; loaded where a stencil asks for it (all 18 first: 87.7
+// us against 79.3 for the whole-list normals at 256^3 FP32, 21.4 against 20.0 at 160^3)
+template <>
+struct PhiNowAt<true> {
+    const Dev* d;
+    int n;
+    __device__ __forceinline__ PhiNowAt(const Dev& dev, int node) : d(&dev), n(node) {}
+    __device__ __forceinline__ double operator()(int a, int b, int c) const { return d->phi[n + a + b * d->L.px + c * d->L.pxy]; }
 };
 
 
