@@ -124,16 +124,7 @@ class Downloader {
                 part(c, t, of);
             }
         };
-        if (nt > 1) {
-            try {
-                threads.reserve(nt - 1);
-                for (int t = 1; t < nt; ++t) threads.emplace_back(worker, t);
-            } catch (const std::exception&) {   // fewer threads than asked for: the parts are cut for those there are
-            }
-        }
-        const int of = (int)threads.size() + 1;
-        team.store(of, std::memory_order_release);
-        int launched = 0;
+        int of = 1, launched = 0;
         for (int c = 0; c < nc && e == hipSuccess; ++c) {
             for (; launched < nc && launched < c + RING && e == hipSuccess; ++launched) {
                 if (launched >= RING)
@@ -145,6 +136,15 @@ class Downloader {
             }
             if (e == hipSuccess) e = hipEventSynchronize(ev[c % RING]);
             if (e != hipSuccess) break;
+            if (c == 0 && nt > 1) {   // the work queued before the download is done: now the threads have something to do
+                try {
+                    threads.reserve(nt - 1);
+                    for (int t = 1; t < nt; ++t) threads.emplace_back(worker, t);
+                } catch (const std::exception&) {   // fewer threads than asked for: the parts are cut for those there are
+                }
+                of = (int)threads.size() + 1;
+                team.store(of, std::memory_order_release);
+            }
             arrived.store(c + 1, std::memory_order_release);
             part(c, 0, of);
         }
