@@ -2099,7 +2099,8 @@ struct mflbm_ctx {
     int device = 0;
     long ps = 0;                // stride of the dense arrays
     double* dense_pdf = nullptr;   // 38 dense arrays: upload/download staging, keeps never-touched slots
-    double* fields = nullptr;   // phi, compact phi, the normal records (4 arrays' worth), curv, u, v, w, rho, phi_old
+    double* phis = nullptr;     // phi, and with a geometry the compact phi behind it (Dev::phic)
+    double* fields = nullptr;   // the normal records (4 arrays' worth), curv, u, v, w, rho, phi_old
     float* fields32 = nullptr;  // FP32 storage modes: the normal records in FP32
     int* role = nullptr;        // dense: fluid boundary index (>= 0) or -(extrapolation list index) - 2, else -1
     unsigned char* qbuf = nullptr;   // brick flags: notm, notp (two buffers each), bstatic, nzb, nzd, hasb
@@ -2526,14 +2527,16 @@ extern "C" int mflbm_create(const mflbm_params* prm, mflbm_ctx** out) {
         return bail(fail(c, MFLBM_ERR_HIP, "hipStreamCreate failed"));
     const long plane = (long)(L.nx + 2) * (L.ny + 2);
     if (hipMalloc(&c->dense_pdf, sizeof(double) * ps * 38) != hipSuccess ||
-        hipMalloc(&c->fields, sizeof(double) * ps * 12) != hipSuccess ||
+        hipMalloc(&c->phis, sizeof(double) * ps) != hipSuccess ||
+        hipMalloc(&c->fields, sizeof(double) * ps * 10) != hipSuccess ||
         hipMalloc(&c->walls, (size_t)ps) != hipSuccess ||
         hipMalloc(&c->planes, sizeof(double) * plane * 40) != hipSuccess ||
         hipMalloc(&c->red, sizeof(double) * (size_t)(L.nz + 1) * 32) != hipSuccess)
         return bail(fail(c, MFLBM_ERR_NOMEM, "device allocation of %.2f GB failed",
-                         (38.0 + 12.0) * 8.0 * ps / 1e9));
+                         (38.0 + 11.0) * 8.0 * ps / 1e9));
     if (hipMemset(c->dense_pdf, 0, sizeof(double) * ps * 38) != hipSuccess ||
-        hipMemset(c->fields, 0, sizeof(double) * ps * 12) != hipSuccess ||
+        hipMemset(c->phis, 0, sizeof(double) * ps) != hipSuccess ||
+        hipMemset(c->fields, 0, sizeof(double) * ps * 10) != hipSuccess ||
         hipMemset(c->walls, 1, (size_t)ps) != hipSuccess || hipMemset(c->planes, 0, sizeof(double) * plane * 40) != hipSuccess)
         return bail(fail(c, MFLBM_ERR_HIP, "hipMemset failed"));
     if (c->fp32 && (hipMalloc(&c->fields32, sizeof(float) * ps * 4) != hipSuccess ||
@@ -2544,16 +2547,15 @@ extern "C" int mflbm_create(const mflbm_params* prm, mflbm_ctx** out) {
         d.cn32 = (float4*)c->fields32;
     }
     d.L = L;
-    d.phi = c->fields;
-    d.phic = c->fields + ps;   // (at most L.total fluid nodes; 2 ps elements stay below 2^32)
-    d.pcoff = (unsigned)ps;
-    d.cn = (double4*)(c->fields + 2 * ps);
-    d.curv = c->fields + 6 * ps;
-    c->u = c->fields + 7 * ps;
-    c->v = c->fields + 8 * ps;
-    c->w = c->fields + 9 * ps;
-    c->rho = c->fields + 10 * ps;
-    c->phi_old = c->fields + 11 * ps;
+    d.phi = c->phis;
+    d.pcoff = (unsigned)ps;   // (at most L.total fluid nodes behind phi: 2 ps elements stay below 2^32)
+    d.cn = (double4*)c->fields;
+    d.curv = c->fields + 4 * ps;
+    c->u = c->fields + 5 * ps;
+    c->v = c->fields + 6 * ps;
+    c->w = c->fields + 7 * ps;
+    c->rho = c->fields + 8 * ps;
+    c->phi_old = c->fields + 9 * ps;
     d.walls = c->walls;
     d.w_in = c->planes;
     d.cphi = c->planes + plane;
@@ -2571,7 +2573,7 @@ extern "C" void mflbm_destroy(mflbm_ctx* c) {
         if (e) (void)hipEventDestroy(e);
     free_geometry(c);
     c->dl.free();
-    void* bufs[] = {c->dense_pdf, c->fields, c->fields32, c->walls, c->planes, c->red};
+    void* bufs[] = {c->dense_pdf, c->phis, c->fields, c->fields32, c->walls, c->planes, c->red};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -2715,6 +2717,16 @@ extern "C" int mflbm_upload_geometry(mflbm_ctx* c, const int8_t* walls_h2, int32
     const long fs = (((long)nfl + 63) / 64) * 64;
     const size_t ni = (size_t)nc + nrm.size() + ns + s1pos.size() + nf + 1;
     const size_t nd = (size_t)ns + s1w.size() + fd.size() + 1;
+    {   // phi moves to an allocation that ends with one value a fluid node; before the others, so that both fit where they do
+        double* phis = nullptr;
+        HIPCHK(c, hipMalloc(&phis, sizeof(double) * (c->ps + (size_t)nfl)));
+        const hipError_t e = hipMemcpy(phis, c->phis, sizeof(double) * c->ps, hipMemcpyDeviceToDevice);
+        (void)hipFree(e == hipSuccess ? c->phis : phis);
+        HIPCHK(c, e);
+        c->phis = c->d.phi = phis;
+        c->d.phic = phis + c->ps;
+        if (nfl > 0) HIPCHK(c, hipMemset(c->d.phic, 0, sizeof(double) * (size_t)nfl));
+    }
     HIPCHK(c, hipMalloc(&c->compact, esz * soff[19]));
     HIPCHK(c, hipMalloc(&c->force, sizeof(double) * fs * 4));
     HIPCHK(c, hipMalloc(&c->map, sizeof(int) * L.total));
@@ -2801,7 +2813,6 @@ extern "C" int mflbm_upload_geometry(mflbm_ctx* c, const int8_t* walls_h2, int32
     HIPCHK(c, hipMemcpy(c->qbuf + 7 * nbr, hasb.data(), nbr, hipMemcpyHostToDevice));
     HIPCHK(c, hipMalloc(&c->cbuf, sizeof(int) * hc.size()));
     HIPCHK(c, hipMemcpy(c->cbuf, hc.data(), sizeof(int) * hc.size(), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemset(c->d.phic, 0, sizeof(double) * (size_t)nfl));
     c->phi_stale = false;
     c->nbricks = (long)nbr;
     c->lcap = lcap;
