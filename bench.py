@@ -479,7 +479,7 @@ def run_nn(args) -> dict:
             "unit": "TFLOP/s", "n_gpus": 1, "dtype": "bf16", "data": "synthetic",
             "roofline": {"bound": "mfma", "achieved": rows[0]["fwd"]["tflops"], "peak": MFMA_BF16_PEAK_TFLOPS,
                          "unit": "TFLOP/s", "frac": rows[0]["fwd"]["frac_of_bf16_peak"], "traffic": None,
-                         "kernel": "k_conv_fwd (level 0: 4 x 64^3, 32 -> 32 channels)"},
+                         "kernel": "k_conv_tile (level 0: 4 x 64^3, 32 -> 32 channels)"},
             "layers": rows}
 
 

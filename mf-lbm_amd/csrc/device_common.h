@@ -42,10 +42,10 @@ __device__ __forceinline__ int xcd_block(int per) { return (int)(blockIdx.x % NX
 // Logical block index of the lattice updates: the dies take runs of UPDATE_RUN consecutive blocks in turn.  In the odd
 // step a slot line is shared by the rows its run boundaries fall on (neighbouring blocks) and read by the planes above
 // and below (some 8 blocks on), so a run keeps most sharers on one die's L2, while all dies still stream one region.
-// Odd step, us, runs of 1 / 8 / 32 / 128 blocks: two-phase 256^3 FP64 665 / 653 / 652 / 685, 160^3 FP32 89 / 85 / 84 /
-// 88, single-phase 160^3 FP64 88 / 81 / 81 / 84 (whole eighths: 88), 125x131x119 FP32 21.7 / 20.0 / 20.0 / 20.1.  The even
-// step shares nothing but finds in its die what the odd step left there: 538 -> 524 us at 256^3, 61 -> 59 and 12.5 -> 11.7
-// us in the single-phase cases, 55 -> 50 us for ten REVs.  The grid is update_grid(blocks).
+// Odd step, us, runs of 1 / 8 / 16 / 32 / 128 blocks: two-phase 256^3 FP64 667 / 651 / 652 / 652 / 685, 160^3 FP32 89 / 85 /
+// 86 / 83 / 88, single-phase 160^3 FP64 88 / 81 / 82 / 82 / 84 (whole eighths: 88), 125x131x119 FP32 21.7 / 19.8 / 19.4 /
+// 19.6 / 20.1: 8 to 32 alike.  The even step shares nothing but finds in its die what the odd step left there (runs of 1 / 16):
+// 538 / 525 us at 256^3, 61 / 60 and 12.5 / 11.8 us in the single-phase cases, 55 / 50 us for ten REVs.  The grid is update_grid(blocks).
 constexpr int UPDATE_RUN = 16;
 __device__ __forceinline__ int update_block() {
     const int x = (int)blockIdx.x % NXCD, i = (int)blockIdx.x / NXCD;

