@@ -754,21 +754,27 @@ extern "C" int mflbm_nn_mfma_probe(const void* a, const void* b, float* d, void*
 
 namespace {
 // Estimated us of the two forward kernels: the latency of a work-group, which grows with the input channels, or, with more
-// work-groups than are in flight at once, so many times it.  Within 25 % of the times measured over d, h, w from 1 to 256.
+// work-groups than the device holds, so many times it; in whole rounds where a compute unit holds one work-group.
+// Fitted to both kernels' times over 240 shapes (sides 1 to 256, 1 to 512 images, 8 to 264 channels in, 8 to 256 out): the
+// kernel that the estimates prefer is within 2 % of the faster one on each, and on 117 random shapes beside them within 3 %
+// but for three of 10 to 17 us (at most 1.4 us).
 // k_conv_fwd: 128 positions x 32 channels a work-group; along an axis one node long a third of the offsets is inside,
 // and a wave skips the loads of the others.
 double untiled_us(const Shape& S, int cin, int cout) {
     const double thin = (S.d == 1 ? 1.0 / 3 : 1.0) * (S.h == 1 ? 1.0 / 3 : 1.0) * (S.w == 1 ? 1.0 / 3 : 1.0);
-    const double groups = (double)((S.count() + 127) / 128) * ((cout + 31) / 32), in_flight = cin >= 64 ? 330 : cin >= 32 ? 560 : 800;
-    return (4.0 + 0.45 * cin) * std::max(0.7 + 0.3 * thin, (0.5 + 0.5 * thin) * groups / in_flight);
+    const double rounds = (double)((S.count() + 127) / 128) * ((cout + 31) / 32) / 256;
+    const double latency = 0.45 * cin * (cin >= 64 ? 1 + cin / 1024.0 * std::min(1.0, rounds) : 1.0);
+    const double round = cin >= 64 ? 0.37 * cin * std::ceil(rounds) : (cin >= 32 ? 0.23 : 0.4) * cin * rounds;
+    return std::max(4.5 + latency * (0.7 + 0.3 * thin), round * (0.5 + 0.5 * thin));
 }
-// k_conv_tile: whole tiles, however much of them lies in the domain; per: us of a work-group per input channel
+// k_conv_tile: whole tiles, however much of them lies in the domain; base and per: us of a work-group and per input channel
 template <int MT, int NCO, int WP, int WC, int TZ, int TY, int TX, int KG>
-double tile_us(const Shape& S, int cin, int cout, double per, double in_flight) {
+double tile_us(const Shape& S, int cin, int cout, double base, double per, double in_flight) {
     using T = ConvTile<MT, NCO, WP, WC, TZ, TY, TX, KG>;
     const double groups = (double)S.n * ((S.d + TZ - 1) / TZ) * ((S.h + TY - 1) / TY) * ((S.w + TX - 1) / TX) * ((cout + T::CO - 1) / T::CO);
     if ((groups + NXCD) * T::THREADS >= 4294967296.0) return HUGE_VAL;   // a launch has less than 2^32 threads
-    return (4.0 + per * cin) * std::max(1.0, groups / in_flight);
+    const double rounds = std::max(1.0, groups / in_flight);
+    return (base + per * cin) * (in_flight == 256 ? std::ceil(rounds) : rounds);
 }
 }  // namespace
 
@@ -789,25 +795,25 @@ extern "C" int mflbm_nn_conv3d_fwd(const void* x, const void* wf, const float* b
     if (cin <= 256 && 10L * h * w * cin * 2 < (1L << 31) && (long)cout * kp * 2 < (1L << 31)) {
         const double tu = untiled_us(S, cin, cout);
         const long tiles8 = (long)n * ((d + 7) / 8) * ((h + 7) / 8) * ((w + 7) / 8);   // 8 x 8 x 8 tiles
-        // PER, FLIGHT: tile_us; then fragments of positions and of channels, waves along positions and channels, tile, steps
-        // per weight stage
-#define TILE_US(PER, FLIGHT, ...) tile_us<__VA_ARGS__>(S, cin, cout, PER, FLIGHT)
-#define TILE(PER, FLIGHT, ...) \
-    if (TILE_US(PER, FLIGHT, __VA_ARGS__) <= tu) return launch_conv_tile<__VA_ARGS__>(x, wf, bias, y, S, (int)cin, (int)cout, kp, (int)relu, st)
+        // BASE, PER, FLIGHT: tile_us; then fragments of positions and of channels, waves along positions and channels, tile,
+        // steps per weight stage
+#define TILE_US(BASE, PER, FLIGHT, ...) tile_us<__VA_ARGS__>(S, cin, cout, BASE, PER, FLIGHT)
+#define TILE(BASE, PER, FLIGHT, ...) \
+    if (TILE_US(BASE, PER, FLIGHT, __VA_ARGS__) <= tu) return launch_conv_tile<__VA_ARGS__>(x, wf, bias, y, S, (int)cin, (int)cout, kp, (int)relu, st)
 #define TILES(BIG, SMALL) \
     if (tiles8 * ((cout + 63) / 64) >= 256 && TILE_US BIG <= TILE_US SMALL) { TILE BIG; } else { TILE SMALL; }
         if (cin <= 32) {   // 4 x 64^3, us before / after: 8 -> 32 75 / 44, 32 -> 8 196 / 85, 32 -> 32 254 / 116, 32 -> 64 483 / 175
-            if (cout <= 16) { TILE(0.15, 400, 2, 1, 8, 1, 4, 8, 8, 8); }
-            else if (cout > 32) { TILE(0.36, 400, 4, 4, 4, 1, 4, 8, 8, 1); }
-            else if (cin <= 16) { TILE(0.19, 400, 4, 2, 4, 1, 4, 8, 8, 4); }
-            else { TILE(0.22, 390, 2, 2, 8, 1, 4, 8, 8, 4); }
+            if (cout <= 16) { TILE(4, 0.15, 300, 2, 1, 8, 1, 4, 8, 8, 8); }
+            else if (cout > 32) { TILE(7, 0.29, 400, 4, 4, 4, 1, 4, 8, 8, 1); }
+            else if (cin <= 16) { TILE(4, 0.19, 400, 4, 2, 4, 1, 4, 8, 8, 4); }
+            else { TILE(4, 0.22, 370, 2, 2, 8, 1, 4, 8, 8, 4); }
         } else if (cin <= 64) {   // 4 x 64^3 64 -> 32 782 / 204; 4 x 32^3 64 -> 64 206 / 46 (61 in the small tile); 4 x 16^3 64 -> 128 52 / 23 (40 in the large)
-            if (cout <= 32) { TILES((0.33, 256, 4, 2, 8, 1, 8, 8, 8, 4), (0.24, 256, 2, 2, 8, 1, 4, 8, 8, 4)) }
-            else { TILES((0.55, 256, 4, 4, 8, 1, 8, 8, 8, 2), (0.25, 256, 2, 2, 4, 2, 4, 4, 8, 4)) }
+            if (cout <= 32) { TILES((4, 0.33, 256, 4, 2, 8, 1, 8, 8, 8, 4), (4, 0.24, 256, 2, 2, 8, 1, 4, 8, 8, 4)) }
+            else { TILES((4, 0.55, 256, 4, 4, 8, 1, 8, 8, 8, 2), (4, 0.25, 256, 2, 2, 4, 2, 4, 4, 8, 4)) }
         } else if (cin <= 128) {   // 4 x 16^3 128 -> 128 100 / 36, 4 x 32^3 128 -> 64 400 / 139
-            TILE(0.22, 256, 2, 2, 4, 2, 4, 4, 8, 8);
+            TILE(4, 0.22, 256, 2, 2, 4, 2, 4, 4, 8, 8);
         } else {   // 4 x 8^3 256 -> 256 125 / 57, 4 x 16^3 256 -> 128 195 / 118
-            TILE(0.2, 256, 1, 2, 4, 2, 4, 4, 4, 4);
+            TILE(4, 0.2, 256, 1, 2, 4, 2, 4, 4, 4, 4);
         }
 #undef TILES
 #undef TILE
